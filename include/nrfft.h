@@ -282,7 +282,9 @@ int nrfft_tune_cache_load(const char* path);
 int nrfft_plan_destroy(nrfft_plan plan);
 /* Bytes of HBM workspace the plan owns. */
 size_t nrfft_plan_workspace_bytes(nrfft_plan plan);
-/* Number of kernel launches one execution enqueues. */
+/* Number of launches of the plan (the range nrfft_execute_c2c_launches indexes).
+ * nrfft_execute_c2c may run both four-step passes of a 1-D plan, all chunks, as
+ * one launch instead (same result up to rounding). */
 int nrfft_plan_num_launches(nrfft_plan plan);
 
 #ifdef __cplusplus

@@ -102,11 +102,28 @@ int get_ctx(DeviceCtx** out) {
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_stage_twiddles, dim3(TW_STAGE_ELEMS / 256), dim3(256), 0, 0, c->c64s, c->c32s);
     HIPCHK(hipGetLastError());
+    HIPCHK(hipMalloc(&c->fs_pool, FS_POOL * sizeof(FsState)));
+    HIPCHK(hipMemset(c->fs_pool, 0, FS_POOL * sizeof(FsState)));
+    c->fs_free.reserve(FS_POOL);
+    for (int i = FS_POOL; i-- > 0;) c->fs_free.push_back(c->fs_pool + i);
     if (int rc = build_mfma_tables(c)) return rc;
     HIPCHK(hipDeviceSynchronize());
     g_ctx[dev] = c;
     *out = c;
     return NRFFT_OK;
+}
+
+FsState* fs_state_take(DeviceCtx* ctx) {
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    if (ctx->fs_free.empty()) return nullptr;
+    FsState* st = ctx->fs_free.back();
+    ctx->fs_free.pop_back();
+    return st;
+}
+void fs_state_give(int device, FsState* st) {
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    auto it = g_ctx.find(device);
+    if (st && it != g_ctx.end()) it->second->fs_free.push_back(st);  // capacity reserved: does not throw
 }
 
 // The current device's context if nrfft_init (or any earlier call) built
@@ -363,6 +380,15 @@ int plan_c2c_1d(Plan& p, int logn, int64_t batch, int src, int dst, size_t* tmp_
         return plan_add_c2c_pass(p, MODE_JJ, logn, 0, d, src, dst);
     }
     if (logn > 2 * C2C_MAX_LOGL_) return fail(NRFFT_E_UNSUPPORTED, "transform longer than 2^26");
+    if (p.fused_ok) {
+        Launch l;
+        size_t ring = 0;
+        if (fused_launch(p, logn, batch, src, dst, FUSED_RING_BYTES, &l, &ring)) {
+            p.launches.push_back(l);
+            *tmp_elems = std::max<size_t>(*tmp_elems, ring);
+            return NRFFT_OK;
+        }
+    }
     // (Split-precision plans keep the two-pass form and its MFMA pass lengths.)
     if (logn >= C2C_3PASS_MIN_LOGN && !(p.kind == PK_C2C && p.extra != 0))
         return plan_c2c_3pass(p, logn, batch, src, dst, tmp_elems);
@@ -387,6 +413,67 @@ int plan_c2c_1d(Plan& p, int logn, int64_t batch, int src, int dst, size_t* tmp_
     }
     p.overlap = overlap;
     return NRFFT_OK;
+}
+
+// Both four-step passes as one launch (k_fused4).  Taken with the default
+// tuning only: an explicit or cached tuning names the split, tiles and chunk
+// of separate passes.
+bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* out,
+                  size_t* ring_elems) {
+    if (p.kind == PK_C2C && p.extra != 0) return false;
+    const size_t n = size_t(1) << logn;
+    if (!(p.tune == default_tune_1d(p.dtype, n, p.batch, 0))) return false;
+    const bool f32 = p.dtype == NRFFT_F32;
+    const FusedRef fp = f32 ? fused_lookup_f32(1, logn) : fused_lookup_f64(1, logn);
+    const FusedRef fm = f32 ? fused_lookup_f32(-1, logn) : fused_lookup_f64(-1, logn);
+    if (!fp.fn || !fm.fn) return false;
+    const int64_t tiles = batch << fp.tiles_log;
+    if (tiles < fused_min_tiles(f32, logn) || tiles >= (int64_t(1) << 30)) return false;
+    DeviceCtx* ctx = nullptr;
+    if (get_ctx(&ctx)) return false;
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fp.fn, FS_NT, 0) != hipSuccess || per_cu < 1) {
+        (void)hipGetLastError();
+        return false;
+    }
+    // Slabs of 64 tiles (8 MiB) or one transform, whichever is larger.
+    Launch l;
+    l.kind = LK_FUSED;
+    l.fn[0] = fp.fn;
+    l.fn[1] = fm.fn;
+    l.src = src;
+    l.dst = dst;
+    l.nt = FS_NT;
+    l.grid = (unsigned)std::min<int64_t>(2 * tiles, int64_t(per_cu) * ctx->ncu);
+    l.fs.batch = (int32_t)batch;
+    l.fs.slab_log = std::max(0, 6 - fp.tiles_log);
+    const int64_t slabs = (batch + (int64_t(1) << l.fs.slab_log) - 1) >> l.fs.slab_log;
+    const size_t slab_elems = n << l.fs.slab_log;
+    const int64_t fit = (int64_t)(ring_bytes / (slab_elems * csize(p.dtype)));
+    const int64_t slots = std::min<int64_t>({slabs, fit, FS_MAX_SLOTS});
+    if (slots < 1 || (slots < 2 && slabs > 1)) return false;
+    l.fs.slots = (int32_t)slots;
+    // Lag: half the ring, but at least 384 tiles (while they fit), so that A
+    // and B tiles both find their counters ready with two groups a CU in
+    // flight.  A ring of less than 1024 tiles that has to be reused feeds one
+    // group a CU at most (64 x 2^20 FP32, 64 MiB ring: 389 us against 496 with
+    // two; 128 MiB: 402 against 361; 192 MiB: 379 against 349).
+    const int64_t slab_tiles = int64_t(1) << (fp.tiles_log + l.fs.slab_log);
+    const int64_t least = std::max<int64_t>(1, 384 / slab_tiles);
+    const bool tight = slots < slabs && slots * slab_tiles < 1024;
+    if (tight) l.grid = std::min(l.grid, (unsigned)ctx->ncu);
+    const int64_t lag = tight ? slots * 3 / 8 : std::max(slots / 2, least);
+    l.fs.lag = (int32_t)std::max<int64_t>(1, std::min(slots - 1, lag));
+    *ring_elems = (size_t)slots * slab_elems;
+    *out = l;
+    return true;
+}
+
+bool plan_is_fused(const Plan& p) {
+    for (const auto* v : {&p.launches, &p.whole})
+        for (const Launch& l : *v)
+            if (l.kind == LK_FUSED) return true;
+    return false;
 }
 
 // Four-step split N = N1 * N2 (x viewed as [n1][n2]) and the two passes'
@@ -522,7 +609,16 @@ int plan_c2c_nd(Plan& p, const std::vector<size_t>& nn, int64_t batch) {
     size_t tmp = 0;
     const size_t ndim = nn.size();
     if (ndim == 1) {
+        const bool fused_ok = p.fused_ok;
+        p.fused_ok = false;
         int rc = plan_c2c_1d(p, ilog2(nn[0]), batch, B_IN, B_OUT, &tmp);
+        p.fused_ok = fused_ok;
+        Launch l;
+        size_t ring = 0;
+        if (!rc && fused_ok && fused_launch(p, ilog2(nn[0]), batch, B_IN, B_OUT, FUSED_RING_BYTES, &l, &ring)) {
+            p.whole.push_back(l);
+            tmp = std::max(tmp, ring);
+        }
         p.tmp_elems = tmp;
         return rc;
     }
@@ -679,7 +775,12 @@ int exec_plan(const Plan& p, const void* in, void* out, void* tmp, const void* a
     if (rc) return rc;
     int idx = -1;
     void* tmp2 = tmp ? static_cast<char*>(tmp) + p.tmp2_offset * csize(p.dtype) : nullptr;
-    void* bufs[B_COUNT] = {const_cast<void*>(in), out, tmp, const_cast<void*>(aux), tmp2, aux2};
+    void* bufs[B_COUNT] = {const_cast<void*>(in), out, tmp, const_cast<void*>(aux), tmp2, aux2, p.fs_state};
+    if (!p.whole.empty() && first == 0 && count < 0) {
+        for (const Launch& l : p.whole)
+            if ((rc = exec_launch(p, l, bufs, isign, stream, ctx))) return rc;
+        return NRFFT_OK;
+    }
     if (p.overlap && first == 0 && count < 0) return exec_overlap(p, bufs, isign, stream, ctx);
     for (const Launch& l : p.launches) {
         ++idx;
@@ -699,6 +800,22 @@ int exec_launch(const Plan& p, const Launch& l, void* const* bufs, int isign, hi
     void* b = static_cast<char*>(bufs[l.dst]) + l.off_dst * (int64_t)csize(p.dtype);
     if (l.kind == LK_COPY) {
         if (a != b) HIPCHK(hipMemcpyAsync(b, a, l.bytes, hipMemcpyDeviceToDevice, stream));
+        return NRFFT_OK;
+    }
+    if (l.kind == LK_FUSED) {
+        FsDesc d = l.fs;
+        void* ring = bufs[B_TMP];
+        void* state = bufs[B_STATE];
+        if (!ring || !state) return fail(NRFFT_E_INVALID, "fused launch without its workspace");
+        if (p.dtype == NRFFT_F32) {
+            Twiddles<float> tw = ctx_twiddles<float>(ctx);
+            void* args[] = {&a, &b, &ring, &state, &d, &tw};
+            HIPCHK(hipLaunchKernel(l.fn[si], dim3(l.grid), dim3(l.nt), args, 0, stream));
+        } else {
+            Twiddles<double> tw = ctx_twiddles<double>(ctx);
+            void* args[] = {&a, &b, &ring, &state, &d, &tw};
+            HIPCHK(hipLaunchKernel(l.fn[si], dim3(l.grid), dim3(l.nt), args, 0, stream));
+        }
         return NRFFT_OK;
     }
     if (l.kind == LK_C2C) {
@@ -825,11 +942,42 @@ int make_plan(nrfft_plan* plan, int kind, int dtype, std::vector<size_t> nn, siz
     p->plan.device = dev;
     if (explicit_tune) p->plan.tune = *explicit_tune;
     else tune_lookup(p->plan);
+    p->plan.fused_ok = true;
     int rc = build_plan(p->plan);
+    // The same plan without fused launches (separate passes, smaller chunks).
+    auto unfused = [&]() {
+        Plan q;
+        q.kind = kind;
+        q.dtype = dtype;
+        q.nn = p->plan.nn;
+        q.batch = batch;
+        q.extra = extra;
+        q.device = dev;
+        q.tune = p->plan.tune;
+        const int r = build_plan(q);
+        if (!r) p->plan = std::move(q);
+        return r;
+    };
+    if (!rc && plan_is_fused(p->plan)) {
+        DeviceCtx* ctx = nullptr;
+        rc = get_ctx(&ctx);
+        if (!rc && !(p->plan.fs_state = fs_state_take(ctx))) rc = unfused();
+    }
     if (!rc && p->plan.tmp_elems) {
         size_t bytes = p->plan.tmp_elems * csize(dtype);
         e = hipMalloc(&p->tmp, bytes);
-        if (e != hipSuccess && kind == PK_C2C && p->plan.nn.size() > 1 && !p->plan.strided_one_pass) {
+        if (e != hipSuccess && p->plan.fs_state) {
+            // No room for the ring of the fused launches.
+            (void)hipGetLastError();
+            fs_state_give(dev, p->plan.fs_state);
+            p->plan.fs_state = nullptr;
+            rc = unfused();
+            if (!rc) {
+                bytes = p->plan.tmp_elems * csize(dtype);
+                e = bytes ? hipMalloc(&p->tmp, bytes) : hipSuccess;
+            }
+        }
+        if (!rc && e != hipSuccess && kind == PK_C2C && p->plan.nn.size() > 1 && !p->plan.strided_one_pass) {
             // The four-step of a long strided axis needs a workspace; without
             // one, such axes run as single column passes.
             (void)hipGetLastError();
@@ -853,6 +1001,7 @@ int make_plan(nrfft_plan* plan, int kind, int dtype, std::vector<size_t> nn, siz
         }
     }
     if (rc) {
+        fs_state_give(dev, p->plan.fs_state);
         delete p;
         return rc;
     }
@@ -996,6 +1145,7 @@ int nrfft_plan_destroy(nrfft_plan plan) {
     g_err.clear();
     if (!plan) return NRFFT_OK;
     if (plan->tmp) (void)hipFree(plan->tmp);
+    fs_state_give(plan->plan.device, plan->plan.fs_state);
     delete plan;
     return NRFFT_OK;
 }

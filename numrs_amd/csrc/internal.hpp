@@ -7,6 +7,7 @@
 #include <functional>
 #include <vector>
 
+#include "fused_c2c.hpp"
 #include "pass_c2c.hpp"
 
 namespace nrfft {
@@ -31,10 +32,13 @@ struct DeviceCtx {
     c32* c32f = nullptr;
     c64* c64s = nullptr;  // per-stage tables (TW_STAGE_ELEMS entries)
     c32* c32s = nullptr;
+    FsState* fs_pool = nullptr;     // FS_POOL counter blocks of fused plans, zeroed
+    std::vector<FsState*> fs_free;  // those no plan holds (guarded by the context lock)
     void* mfma_f16 = nullptr;   // split-precision DFT-matrix operands
     void* mfma_bf16 = nullptr;
     int ncu = 256;        // compute units
 };
+constexpr int FS_POOL = 256;  // at most so many fused plans on a device at a time (2 MiB)
 int build_mfma_tables(DeviceCtx* c);
 const KernelRef& mfma_lookup(int prec, int sign, int mode, int logl);
 template <typename T>
@@ -50,7 +54,8 @@ int noalloc_setup(int device);
 
 // Buffers a launch reads or writes.
 // B_AUX2: a second caller buffer (twofft's second spectrum, rlft3's speq).
-enum BufId { B_IN = 0, B_OUT = 1, B_TMP = 2, B_AUX = 3, B_TMP2 = 4, B_AUX2 = 5, B_COUNT = 6 };
+// B_STATE: the counters of fused launches (FsState, zero between launches).
+enum BufId { B_IN = 0, B_OUT = 1, B_TMP = 2, B_AUX = 3, B_TMP2 = 4, B_AUX2 = 5, B_STATE = 6, B_COUNT = 7 };
 // Plan kinds.
 enum PlanKind {
     PK_C2C = 0,
@@ -64,7 +69,7 @@ enum PlanKind {
     PK_UNEVEN = 8  // tune-cache key of an uneven-batch size class (nn = {N}, batch 0)
 };
 // Launch kinds.
-enum LaunchKind { LK_C2C = 0, LK_COPY = 1, LK_REAL = 2, LK_SPEC = 3 };
+enum LaunchKind { LK_C2C = 0, LK_COPY = 1, LK_REAL = 2, LK_SPEC = 3, LK_FUSED = 4 };
 
 // Tunables chosen per (kind, N, batch, dtype); -1 = default.
 struct Tune {
@@ -90,6 +95,7 @@ struct Launch {
     int ti = 0;
     int mode = 0;
     PassDesc desc{};
+    FsDesc fs{};          // LK_FUSED
     int src = B_IN;
     int dst = B_OUT;
     int prec = 0;         // 0 = plain kernel, else split-precision MFMA kernel (MfmaPrec)
@@ -118,6 +124,15 @@ struct Plan {
     int device = 0;
     Tune tune;
     std::vector<Launch> launches;
+    // When not empty, what a whole execution enqueues instead of `launches`
+    // (a 1-D C2C plan whose two passes run as one fused launch; the
+    // pass-by-pass form stays for nrfft_execute_c2c_launches).
+    std::vector<Launch> whole;
+    // The plan has counters of its own (fs_state_take), so four-step transforms
+    // may run as fused launches.  False for the host-pointer calls' plans, which
+    // several calls may execute at once.
+    bool fused_ok = false;
+    FsState* fs_state = nullptr;
     size_t tmp_elems = 0;    // complex elements of workspace
     size_t tmp2_offset = 0;  // B_TMP2 = workspace + tmp2_offset complex elements
     // Strided n-D axes of >= 4096 points run as one column pass (no
@@ -191,6 +206,33 @@ int plan_c2c_mapped(Plan& p, int logn, int64_t batch, int src, int dst, int lmap
 // lmap: a four-step length whose first pass has a load-mapped kernel of the
 // plan's tile width.
 bool map_fits(const Plan& p, int logn, int lmap);
+// A kernel of both four-step passes (k_fused4), fn == nullptr if there is none.
+struct FusedRef {
+    const void* fn;
+    int tiles_log;  // log2 tiles of one pass per transform
+};
+FusedRef fused_lookup_f32(int sign, int logn);
+FusedRef fused_lookup_f64(int sign, int logn);
+// The fused launch of `batch` transforms of 2^logn points from src to dst
+// with a ring of at most ring_bytes; false if the size has no such kernel or
+// runs faster as separate passes.  *ring_elems: complex values of its ring.
+bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* l,
+                  size_t* ring_elems);
+// Fewest tiles of a pass for the fused launch (its lead-in and its tail run
+// one pass only).  MI355X, buffers changing from call to call, fused against
+// separate passes: FP32 2^20 640 tiles 68.7 / 74.9 us, 512 tiles 58.7 / 60.1,
+// 384 tiles 52.1 / 47.8; FP32 2^15 640 tiles 66.7 / 67.2; FP64 2^16 640 tiles
+// 63.7 / 68.3; FP64 2^18 768 tiles 74.9 / 75.9, 640 tiles 67.2 / 64.1.
+inline int64_t fused_min_tiles(bool f32, int logn) { return !f32 && logn >= 18 ? 1024 : 640; }
+constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;
+bool plan_is_fused(const Plan& p);
+// A zeroed FsState of the current device's pool for a plan with fused
+// launches (nullptr: none left), and its return.  A launch leaves its counters
+// zero, so a returned state is ready for the next plan once the launches of
+// the last one are done (destroying a plan frees its workspace, which waits
+// for them).
+FsState* fs_state_take(DeviceCtx* ctx);
+void fs_state_give(int device, FsState* st);
 int exec_launch(const Plan& p, const Launch& l, void* const* bufs, int isign, hipStream_t stream, DeviceCtx* ctx);
 int col_tilog(int dtype);
 int exec_plan(const Plan& p, const void* in, void* out, void* tmp, const void* aux, int isign, hipStream_t stream,

@@ -26,12 +26,21 @@
 #endif
 
 static __device__ __align__(256) unsigned char scratch[NRFFT_NOALLOC_SCRATCH_BYTES];
+// Counters of the fused launches (k_fused4), cleared before each: calls that
+// raced may have left them anyhow.
+static __device__ nrfft::FsState fused_state;
 
 namespace nrfft {
+
+__global__ void k_fused_clear(FsState* st) {
+    uint32_t* p = reinterpret_cast<uint32_t*>(st);
+    for (unsigned i = threadIdx.x; i < sizeof(FsState) / 4; i += blockDim.x) p[i] = 0;
+}
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static std::mutex g_scratch_mu;
 static void* g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
+static void* g_fused_state_ptr[NOALLOC_MAX_DEVICES] = {};
 
 int noalloc_setup(int device) {
     if (device < 0 || device >= NOALLOC_MAX_DEVICES) return fail(NRFFT_E_INVALID, "device index out of range");
@@ -41,15 +50,21 @@ int noalloc_setup(int device) {
     const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
     if (e != hipSuccess || !ptr)
         return fail(NRFFT_E_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
+    void* st = nullptr;
+    const hipError_t es = hipGetSymbolAddress(&st, HIP_SYMBOL(fused_state));
+    if (es != hipSuccess || !st)
+        return fail(NRFFT_E_HIP, std::string("hipGetSymbolAddress(fused_state): ") + hipGetErrorString(es));
     g_scratch_ptr[device] = ptr;
+    g_fused_state_ptr[device] = st;
     return NRFFT_OK;
 }
 
-static int scratch_of(int device, void** out) {
+static int scratch_of(int device, void** out, void** state) {
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     if (device < 0 || device >= NOALLOC_MAX_DEVICES || !g_scratch_ptr[device])
         return fail(NRFFT_E_INVALID, "nrfft_init(" + std::to_string(device) + ") has not run on this device");
     *out = g_scratch_ptr[device];
+    *state = g_fused_state_ptr[device];
     return NRFFT_OK;
 }
 
@@ -72,8 +87,8 @@ static int noalloc_c2c(int dtype, const void* d_in, void* d_out, size_t nn, size
     if (hipGetDevice(&dev) != hipSuccess) return fail(NRFFT_E_HIP, "hipGetDevice");
     DeviceCtx* ctx = nullptr;
     if (int rc = find_ctx(&ctx)) return rc;
-    void* ws = nullptr;
-    if (int rc = scratch_of(dev, &ws)) return rc;
+    void *ws = nullptr, *state = nullptr;
+    if (int rc = scratch_of(dev, &ws, &state)) return rc;
     // A host-side plan description on the stack (its vectors stay empty).
     Plan p;
     p.kind = PK_C2C;
@@ -81,7 +96,7 @@ static int noalloc_c2c(int dtype, const void* d_in, void* d_out, size_t nn, size
     p.batch = batch;
     p.device = dev;
     p.tune = default_tune_1d(dtype, nn, batch, 0);
-    void* bufs[B_COUNT] = {const_cast<void*>(d_in), d_out, ws, nullptr, nullptr, nullptr};
+    void* bufs[B_COUNT] = {const_cast<void*>(d_in), d_out, ws, nullptr, nullptr, nullptr, state};
     const int64_t N = int64_t(nn);
     if (logn == 0) {
         if (d_in != d_out && hipMemcpyAsync(d_out, d_in, batch * cs, hipMemcpyDeviceToDevice, stream) != hipSuccess)
@@ -102,6 +117,13 @@ static int noalloc_c2c(int dtype, const void* d_in, void* d_out, size_t nn, size
         Launch l;
         if (int rc = c2c_pass_launch(p, MODE_JJ, logn, 0, d, B_IN, B_OUT, &l)) return rc;
         return exec_launch(p, l, bufs, isign, stream, ctx);
+    }
+    Launch fused;
+    size_t ring = 0;
+    if (fused_launch(p, logn, (int64_t)batch, B_IN, B_OUT, NRFFT_NOALLOC_SCRATCH_BYTES, &fused, &ring)) {
+        hipLaunchKernelGGL(k_fused_clear, dim3(1), dim3(256), 0, stream, (FsState*)state);
+        if (hipGetLastError() != hipSuccess) return fail(NRFFT_E_HIP, "k_fused_clear");
+        return exec_launch(p, fused, bufs, isign, stream, ctx);
     }
     FourStep fs;
     if (int rc = fourstep_setup(p, logn, &fs)) return rc;

@@ -389,7 +389,7 @@ int build_plan_real(Plan& p) {
     // Both forward spectra use isign = +1 whatever isign the call carries
     // (for convlv isign selects convolution or deconvolution).
     for (auto& l : p.launches)
-        if (l.kind == LK_C2C) l.args[6] = 1;
+        if (l.kind == LK_C2C || l.kind == LK_FUSED) l.args[6] = 1;
     p.launches.push_back(real_launch(RS_SPEC, B_OUT, B_OUT, {batch, L, NRFFT_SPEC_RAW ? 1 : 0}));
     // The inverse C2C of the last step runs with isign = -1 whatever isign
     // the call carries (isign selects conv/deconv); args[6] marks it.

@@ -170,6 +170,7 @@ static std::vector<Tune> candidates(int dtype, const std::vector<size_t>& nn, si
     if (nn.size() == 1) {
         const int logn = ilog2(nn[0]);
         if (logn <= C2C_MAX_LOGL_) return {Tune{}};
+        out.push_back(default_tune_1d(dtype, nn[0], batch, 0));  // (the only one that may run as a fused launch)
         std::vector<int> chunks = {0};
         for (int c = 1; c < (int)batch; c *= 2) chunks.push_back(c);
         for (int l1 = std::max(1, logn - C2C_MAX_LOGL_); l1 <= std::min(C2C_MAX_LOGL_, logn - 1); ++l1) {
@@ -197,11 +198,18 @@ static std::vector<Tune> candidates(int dtype, const std::vector<size_t>& nn, si
     return out;
 }
 
-static int time_plan(const Plan& p, void* in, void* out, int iters, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
+static int time_plan(Plan& p, void* in, void* out, int iters, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
                      float* ms) {
     void* tmp = nullptr;
     if (p.tmp_elems) {
         if (hipMalloc(&tmp, p.tmp_elems * csize(p.dtype)) != hipSuccess) return NRFFT_E_NOMEM;
+    }
+    if (plan_is_fused(p)) {
+        DeviceCtx* ctx = nullptr;
+        if (get_ctx(&ctx) || !(p.fs_state = fs_state_take(ctx))) {
+            (void)hipFree(tmp);
+            return NRFFT_E_NOMEM;
+        }
     }
     int rc = NRFFT_OK;
     for (int w = 0; w < 2 && !rc; ++w) rc = exec_plan(p, in, out, tmp, nullptr, 1, s);
@@ -216,6 +224,8 @@ static int time_plan(const Plan& p, void* in, void* out, int iters, hipStream_t 
     }
     (void)hipStreamSynchronize(s);
     if (tmp) (void)hipFree(tmp);
+    fs_state_give(p.device, p.fs_state);
+    p.fs_state = nullptr;
     return rc;
 }
 
@@ -282,6 +292,8 @@ int nrfft_autotune_c2c(int dtype, const size_t* nn, size_t ndim, size_t batch, i
             p.nn = d;
             p.batch = batch;
             p.tune = t;
+            p.fused_ok = true;
+            (void)hipGetDevice(&p.device);
             if (build_plan(p) != NRFFT_OK) continue;
             float ms = 0;
             if (time_plan(p, in, out, iters, s, e0, e1, &ms) != NRFFT_OK) continue;
