@@ -11,10 +11,10 @@
 // each point once in and once out, the last-level cache (MALL) the
 // intermediate once in and once out; a copy kernel with these four streams,
 // this tile shape and this ticket order takes 297 us for 64 x 2^20 FP32 on
-// MI355X (random data; 2 GiB past the L2s, 7.2 TB/s), this kernel 336.  Two
+// MI355X (random data; 2 GiB past the L2s, 7.2 TB/s), this kernel 324.  Two
 // launches per batch chunk (k_c2c_dma / k_c2c) took 445: each pays a ramp and a
 // drain, and their chunks have to be 64-128 MiB to fill the chip, so input,
-// intermediate and output share the MALL.  FP64 45 x 2^18 150 -> 128 us.
+// intermediate and output share the MALL.  FP64 45 x 2^18 150 -> 126 us.
 //
 // Groups take work from one ticket counter.  A ticket is a unit: A tile u,
 // then B tile u - lead, with lead = `lag` slabs; a slab is 64 tiles
@@ -32,11 +32,14 @@
 // tiles of the slab that was there have all loaded.  A tile depends only on
 // units with smaller tickets, and a group that holds a ticket runs, so the
 // smallest unfinished unit never waits: no deadlock, however few groups are
-// resident.  Every wait is bounded all the same (FS_SPIN polls), so misuse
-// (one plan on two streams at once) gives wrong results, not a hang.
+// resident.  Every wait is bounded all the same (a group polls FS_SPIN times in
+// vain at most once), so misuse (one plan on two streams at once) gives wrong
+// results, not a hang.
 //
 // The last group to leave clears the counters, so a launch leaves the state
-// as it found it and needs no reset launch or memset before it.
+// as it found it and needs no reset launch or memset before it.  (The count of
+// groups that have left is taken down by the launch's own: whatever overlapped,
+// the very last group finds the others gone and clears everything.)
 #pragma once
 #include "pass_c2c.hpp"
 
@@ -125,50 +128,79 @@ __device__ __forceinline__ void fs_dft(cpx<T>* v) {
     else dft<R, S>(v);
 }
 
-// Radix plan: two stages (one exchange) where the values per thread allow
-// it, else the plan of RadixPlan (whose last stage's twiddles are then read
-// from the global per-stage table).
+// Radix plan of a tile's transforms: two stages (one exchange) where the
+// values per thread allow it, else the plan of RadixPlan (stages from the third
+// on read the global per-stage table).
+template <int... RS>
+struct FsRadices {
+    static constexpr int NST = sizeof...(RS);
+    static constexpr int R[NST] = {RS...};
+};
+template <int L>
+using FsTablePlan = std::conditional_t<
+    RadixPlan<L>::NST == 2, FsRadices<RadixPlan<L>::radix(0), RadixPlan<L>::radix(1)>,
+    std::conditional_t<RadixPlan<L>::NST == 3,
+                       FsRadices<RadixPlan<L>::radix(0), RadixPlan<L>::radix(1), RadixPlan<L>::radix(2)>,
+                       FsRadices<RadixPlan<L>::radix(0), RadixPlan<L>::radix(1), RadixPlan<L>::radix(2),
+                                 RadixPlan<L>::radix(3)>>>;
 template <typename T, int L>
-struct FsPlan;
-template <> struct FsPlan<float, 128> { static constexpr int NST = 2, R[3] = {8, 16, 1}; };
-template <> struct FsPlan<float, 256> { static constexpr int NST = 2, R[3] = {16, 16, 1}; };
-template <> struct FsPlan<float, 512> { static constexpr int NST = 2, R[3] = {16, 32, 1}; };
-template <> struct FsPlan<float, 1024> { static constexpr int NST = 2, R[3] = {32, 32, 1}; };
-template <> struct FsPlan<float, 2048> { static constexpr int NST = 3, R[3] = {8, 16, 16}; };
-template <> struct FsPlan<double, 128> { static constexpr int NST = 2, R[3] = {8, 16, 1}; };
-template <> struct FsPlan<double, 256> { static constexpr int NST = 2, R[3] = {16, 16, 1}; };
-template <> struct FsPlan<double, 512> { static constexpr int NST = 3, R[3] = {2, 16, 16}; };
-template <> struct FsPlan<double, 1024> { static constexpr int NST = 3, R[3] = {4, 16, 16}; };
+struct FsPlan : FsTablePlan<L> {};
+template <typename T> struct FsPlan<T, 64> : FsRadices<8, 8> {};
+template <> struct FsPlan<float, 512> : FsRadices<16, 32> {};
+template <> struct FsPlan<float, 1024> : FsRadices<32, 32> {};
+
+// Stage-1 twiddle rows in LDS: entry (k, r) at p[k ROW_ + r COL_].
+template <typename T, int ROW_, int COL_>
+struct FsLtw {
+    static constexpr int ROW = ROW_, COL = COL_;
+    const cpx<T>* p;
+};
 
 // ---------------------------------------------------------------------------
 // Stage engine of one tile: EPT values per thread.  Stage 0 is mapped along
-// (MAP_J) or across (MAP_T) the transforms, later stages across.  The exchanges
+// (MAP_J) or across (MAP_T) the transforms, later stages by MAPS.  The exchanges
 // move one real component at a time, so a tile needs half the LDS and two
 // groups share a CU: one's loads and stores run under the other's arithmetic.
-// LDS layout [i][TI] with gaps that keep the first exchange's writes in
-// distinct banks (the accesses of LANES lanes meet in the banks):
-//   MAP_T  LANES holds G = LANES / TI butterflies j; they are taken G apart
-//          (j = (jj mod G) L / (R0 G) + jj / G, jj = thread / TI), and each of
-//          the G parts of the tile is moved on by TI values;
-//   MAP_J  lanes along j write R0 TI apart: a gap after every R0 TI values.
-// Reads and the second exchange's writes take consecutive addresses.
+// LDS layout with gaps that keep the first exchange's writes in distinct
+// banks (LANES lanes meet in the banks); elements of a transform are
+//   MAPS = MAP_T  TI apart ([i][TI]).  Lanes across the transforms (MAPL =
+//          MAP_T): LANES holds G = LANES / TI (at most 16) butterflies j; they
+//          are taken L / (R0 G) apart (j = (jj mod G) L / (R0 G) + jj / G, jj =
+//          thread / TI), and each of the G parts of the tile is moved on by TI
+//          values.  Lanes along j (MAPL = MAP_J) write R0 TI apart: a gap after
+//          every R0 TI values.
+//   MAPS = MAP_J  contiguous ([t][L]), a gap of one after every LANES values.
+// Reads and the later exchanges' writes take (nearly) consecutive addresses.
 // ---------------------------------------------------------------------------
-template <typename T, int S, int L, int MAPL>
+template <typename T, int S, int L, int MAPL, int MAPS = MAP_T>
 struct FsEng {
+    static_assert(MAPS == MAP_T || MAPL == MAP_J, "row stores come with row loads");
     using P = FsPlan<T, L>;
     static constexpr int EPT = fs_ept<T>(), NT = FS_NT, TI = fs_tile<T>() / L, NST = P::NST;
     static constexpr int R0 = P::R[0];
-    static constexpr int ns(int s) { return s == 0 ? 1 : s == 1 ? P::R[0] : P::R[0] * P::R[1]; }
+    static constexpr int ns(int s) {
+        int n = 1;
+        for (int q = 0; q < s; ++q) n *= P::R[q];
+        return n;
+    }
     static constexpr int RL = P::R[NST - 1];   // last radix
     static constexpr int NBL = L / RL;         // output k = j + r NBL
     static constexpr int LANES = 256 / (int)sizeof(T);
-    static constexpr int G = (MAPL == MAP_T && TI < LANES) ? LANES / TI : 1;
-    static constexpr int BLK = MAPL == MAP_T ? TI * L / G : R0 * TI;
-    static constexpr int PADQ = MAPL == MAP_T ? (G > 1 ? TI : 0) : (L / R0 >= LANES ? 1 : LANES / (L / R0));
+    static constexpr bool COLS = MAPL == MAP_T;  // stage 0 across the transforms
+    static constexpr int G = (COLS && TI < LANES) ? (LANES / TI < 16 ? LANES / TI : 16) : 1;
+    static constexpr int TS = MAPS == MAP_T ? TI : 1;  // distance of neighbouring elements
+    static constexpr int BLK = MAPS == MAP_J ? LANES : COLS ? TI * L / G : R0 * TI;
+    static constexpr int PADQ = MAPS == MAP_J ? 1 : COLS ? (G > 1 ? TI : 0) : (L / R0 >= LANES ? 1 : LANES / (L / R0));
     static constexpr int EX_ELEMS = TI * L + (TI * L / BLK) * PADQ;
-    static_assert(G == 1 || (P::R[1] % G == 0 && (L / R0) % G == 0 && (NST < 3 || P::R[2] % G == 0)),
-                  "gaps fall on whole radix steps");
+    static constexpr bool parts_whole() {
+        if (G == 1) return true;
+        for (int s = 1; s < NST; ++s)
+            if (P::R[s] % G) return false;
+        return (L / R0) % G == 0;
+    }
+    static_assert(parts_whole(), "gaps fall on whole radix steps");
     static constexpr int phys(int raw) { return raw + raw / BLK * PADQ; }
+    static __device__ __forceinline__ int raw_of(int t, int i) { return MAPS == MAP_T ? i * TI + t : t * L + i; }
 
     template <int s, class F>
     static __device__ __forceinline__ void each_butterfly(int tid, F&& f) {
@@ -178,7 +210,7 @@ struct FsEng {
         for (int b = 0; b < BPT; ++b) {
             const unsigned q = unsigned(tid) + unsigned(b * NT);
             int t, j;
-            if constexpr (s == 0 && MAPL == MAP_J) {
+            if constexpr ((s == 0 ? MAPL : MAPS) == MAP_J) {
                 t = int(q / unsigned(NB));
                 j = int(q % unsigned(NB));
             } else {
@@ -195,31 +227,35 @@ struct FsEng {
     static __device__ __forceinline__ void put(const cpx<T>* v, int tid, T* ex) {
         constexpr int R = P::R[s], NS = ns(s);
         each_butterfly<s>(tid, [&](int b, int t, int j) {
-            T* base = ex + phys(((j / NS) * NS * R + (j % NS)) * TI + t);
-            // A butterfly's outputs lie in one gap-free part (MAP_T; MAP_J,
-            // s = 0), or one part apart each (MAP_J, s = 1: NS TI = BLK).
-            constexpr int step = NS * TI + (MAPL == MAP_J && s > 0 ? PADQ : 0);
+            T* base = ex + phys(raw_of(t, (j / NS) * NS * R + (j % NS)));
+            // Columns: a butterfly's outputs lie in one gap-free part.  Rows in,
+            // columns out: R0 of them do (s = 0), or they lie whole parts apart.
+            // Rows: at compile-time distances (NS divides LANES or is a multiple).
 #pragma unroll
-            for (int r = 0; r < R; ++r) base[r * step] = C == 0 ? v[b * R + r].x : v[b * R + r].y;
+            for (int r = 0; r < R; ++r) {
+                const int o = r * NS * TS + (MAPS == MAP_J ? r * NS / LANES : COLS || s == 0 ? 0 : r * (NS / R0) * PADQ);
+                base[o] = C == 0 ? v[b * R + r].x : v[b * R + r].y;
+            }
         });
     }
     template <int s, int C>
     static __device__ __forceinline__ void get(cpx<T>* v, int tid, const T* ex) {
         constexpr int R = P::R[s], NB = L / R;
         each_butterfly<s>(tid, [&](int b, int t, int j) {
-            // element j + r NB: r alone says in which part it lies (MAP_T), or
-            // NB TI is a multiple of BLK (MAP_J)
-            const T* base = ex + (MAPL == MAP_T ? j * TI + t : phys(j * TI + t));
+            // element j + r NB: r alone says in which part it lies (columns), or
+            // r NB TS / BLK is its share of the gaps
+            const T* base = ex + (COLS ? j * TI + t : phys(raw_of(t, j)));
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const int o = r * NB * TI + (r * NB * TI) / BLK * PADQ;
+                const int o = r * NB * TS + (r * NB * TS) / BLK * PADQ;
                 if constexpr (C == 0) v[b * R + r].x = base[o];
                 else v[b * R + r].y = base[o];
             }
         });
     }
-    // Stage 1's twiddles come from LDS (NS rows of R + 2 entries, W_{NS R}^{r k},
-    // exact entries of the coarse table), stage 2's from the per-stage table.
+    // Stage 1's twiddles W_{NS R}^{r k} come from LDS (FsLtw: rows k; by default NS
+    // rows of R + 2 entries, exact entries of the coarse table), later ones from
+    // the per-stage table.
     static constexpr int TW_ELEMS = ns(1) * (P::R[1] + 2);
     static __device__ __forceinline__ void fill_tw(cpx<T>* ltw, const cpx<T>* coarse, int tid) {
         constexpr int R = P::R[1], NS = ns(1);
@@ -228,14 +264,15 @@ struct FsEng {
             ltw[k * (R + 2) + r] = coarse[(r * k) * (TW_COARSE / (NS * R))];
         }
     }
-    template <int s>
-    static __device__ __forceinline__ void twiddle(cpx<T>* v, int tid, const cpx<T>* ltw, const cpx<T>* stage_tw) {
-        constexpr int R = P::R[s], NS = ns(s);
+    using Ltw = FsLtw<T, P::R[1] + 2, 1>;
+    template <int s, class LTW>
+    static __device__ __forceinline__ void twiddle(cpx<T>* v, int tid, LTW ltw, const cpx<T>* stage_tw) {
+        constexpr int R = P::R[s], NS = ns(s), RS = s == 1 ? LTW::COL : 1;
         each_butterfly<s>(tid, [&](int b, int, int j) {
-            const cpx<T>* row = s == 1 ? ltw + (j % NS) * (R + 2)
+            const cpx<T>* row = s == 1 ? ltw.p + (j % NS) * LTW::ROW
                                        : stage_tw + 2 * L + StageTable<L>::off(s) + (j % NS) * R;
 #pragma unroll
-            for (int r = 1; r < R; ++r) v[b * R + r] = cmul(v[b * R + r], dirw<S>(row[r]));
+            for (int r = 1; r < R; ++r) v[b * R + r] = cmul(v[b * R + r], dirw<S>(row[r * RS]));
         });
     }
     template <int s>
@@ -244,18 +281,18 @@ struct FsEng {
 #pragma unroll
         for (int b = 0; b < EPT / R; ++b) fs_dft<R, S>(v + b * R);
     }
-    // Stages 1 .. NST-1; stage 0's outputs are in v.  `mid` runs after the
-    // first barrier, `late` before the last stage.
-    template <int s = 1, class MID, class LATE>
-    static __device__ __forceinline__ void rest(cpx<T>* v, int tid, T* ex, const cpx<T>* ltw, const cpx<T>* stage_tw,
+    // Stages 1 .. NST-1; stage 0's outputs are in v.  Hooks in the last exchange:
+    // `pre` before it, `mid` behind its first barrier, `late` before its last read.
+    template <int s = 1, class LTW, class PRE, class MID, class LATE>
+    static __device__ __forceinline__ void rest(cpx<T>* v, int tid, T* ex, LTW ltw, const cpx<T>* stage_tw, PRE&& pre,
                                                 MID&& mid, LATE&& late) {
-        static_assert(NST == 2 || (RadixPlan<L>::NST == 3 && RadixPlan<L>::radix(2) == P::R[2] &&
-                                   RadixPlan<L>::ns(2) == ns(2)), "stage 2 reads the per-stage table");
+        static_assert(NST == 2 || std::is_base_of_v<FsTablePlan<L>, P>, "stage 2 reads the per-stage table");
         if constexpr (s < NST) {
             if constexpr (s > 1) lds_barrier();  // the previous exchange has been read
+            if constexpr (s == NST - 1) pre();
             put<s - 1, 0>(v, tid, ex);
             lds_barrier();
-            if constexpr (s == 1) mid();
+            if constexpr (s == NST - 1) mid();
             get<s, 0>(v, tid, ex);
             lds_barrier();
             put<s - 1, 1>(v, tid, ex);
@@ -264,7 +301,7 @@ struct FsEng {
             get<s, 1>(v, tid, ex);
             twiddle<s>(v, tid, ltw, stage_tw);
             butterflies<s>(v);
-            rest<s + 1>(v, tid, ex, ltw, stage_tw, mid, late);
+            rest<s + 1>(v, tid, ex, ltw, stage_tw, pre, mid, late);
         }
     }
 };
@@ -274,7 +311,9 @@ struct FsEng {
 // = W^{n2 (j + 4 h NB)}, b[l] = W^{n2 l NB}.  Every second a[h] and the b[l]
 // (FP64: b[1], b[2]) are table products, so a factor is at most three products
 // away from them.
-// The table values are loaded before the exchange and joined after it.
+// The table values are loaded before the last exchange and joined behind its
+// first barrier: loaded with the tile they took 32 registers through the first
+// stages (64 x 2^20 FP32 337 us against 324, FP64 2^19 and 2^20 spilled).
 template <typename T, int S, int R, int BPT, int NB>
 struct FsTw {
     static_assert(R >= 8 && R % 8 == 0, "last radix 8, 16 or 32");
@@ -435,6 +474,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
     const bool wave0 = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
     uint32_t taken = 0;            // lane 0: the ticket as it arrives
     uint32_t next = 0, seen = 0;   // wave 0: the coming task, and its counter as last read
+    int patience = FS_SPIN;        // polls
     uint32_t* pending = nullptr;   // counter of the group's last A tile, its stores perhaps in flight
     // (Through a pointer the compiler must take for lane-dependent: for a
     // uniform one it broadcasts the result at once, i.e. waits for the atomic
@@ -478,10 +518,12 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             if (wave0) {
                 const uint32_t* p = waits_on(t);
                 const uint32_t need = need_of(t);
-                for (int i = 0; i < FS_SPIN; ++i) {
+                int i = 0;
+                for (; i < patience; ++i) {
                     if (__builtin_amdgcn_readfirstlane(fs_peek(p)) >= need) break;
                     __builtin_amdgcn_s_sleep(8);
                 }
+                if (i == patience) patience = 0;
             }
             lds_barrier();
         }
@@ -514,17 +556,26 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             publish();
             if (last_of_unit(k)) take_ticket();
             FsTw<T, S, EA::RL, EPT / EA::RL, EA::NBL> f;
-            {
+            auto load_tw = [&]() {
                 uint32_t n2 = 0, jl[EPT / EA::RL];
                 EA::template each_butterfly<EA::NST - 1>(ltid, [&](int b, int tt, int j) {
                     n2 = idx * uint32_t(TA) + uint32_t(tt);  // the same for every b
                     jl[b] = uint32_t(j);
                 });
                 f.load(tw, n2, jl, LOGN);
-            }
+            };
             __builtin_amdgcn_s_setprio(1);
             EA::template butterflies<0>(v);
-            EA::rest(v, ltid, ex, ltwa, tw.stage, [&]() { __builtin_amdgcn_s_setprio(2); f.join(); }, [&]() { look(k); __builtin_amdgcn_s_setprio(3); });
+            EA::rest(
+                v, ltid, ex, typename EA::Ltw{ltwa}, tw.stage, load_tw,
+                [&]() {
+                    __builtin_amdgcn_s_setprio(2);
+                    f.join();
+                },
+                [&]() {
+                    look(k);
+                    __builtin_amdgcn_s_setprio(3);
+                });
             f.apply(v);
             // ring: [block b = k1 / TB][block a = idx][k1 mod TB][n2 mod TA]
             const __amdgpu_buffer_rsrc_t rr = fs_rsrc(rt, uint32_t(N * CS));
@@ -561,7 +612,12 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                 arrive[1] = 0;
                 fs_count(st->loaded[t.slot]);
             }
-            EB::rest(v, ltid, ex, ltwb, tw.stage, [&]() { __builtin_amdgcn_s_setprio(2); }, [&]() { look(k); __builtin_amdgcn_s_setprio(3); });
+            EB::rest(
+                v, ltid, ex, typename EB::Ltw{ltwb}, tw.stage, []() {}, []() { __builtin_amdgcn_s_setprio(2); },
+                [&]() {
+                    look(k);
+                    __builtin_amdgcn_s_setprio(3);
+                });
             const __amdgpu_buffer_rsrc_t ro = fs_rsrc(out + int64_t(tr) * N, uint32_t(N * CS));
             EB::template each_butterfly<EB::NST - 1>(ltid, [&](int b, int tt, int j) {
                 constexpr int R = EB::RL, NB = EB::NBL;
@@ -592,7 +648,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
         }
         if (tid == 0) {
             __hip_atomic_store(&st->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&st->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_sub(&st->done, gridDim.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
