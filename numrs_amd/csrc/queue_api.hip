@@ -28,13 +28,18 @@ struct UnevenItem {
 struct UnevenState {
     int dtype = 0;
     std::vector<UnevenItem> items;
-    std::vector<QTask> tasks;  // phase 1 then phase 2
-    int n1 = 0, n2 = 0;
-    size_t ws_elems = 0;
+    std::vector<QTask> tasks;  // in the order in which they are taken, two to a ticket
+    int n1 = 0, n2 = 0;        // single- and first-pass tiles, second-pass tiles
+    std::vector<uint32_t> offs;  // of the items of single-pass tiles, from their tile's base
+    bool few = false;          // one group per CU
+    std::vector<uint32_t> init;  // the counters' initial values
+    size_t ring_elems = 0;
     size_t total_elems = 0;
     QTask* d_tasks = nullptr;
-    QState* d_state = nullptr;
-    void* d_ws = nullptr;
+    uint32_t* d_offs = nullptr;
+    uint32_t* d_init = nullptr;
+    uint32_t* d_ctr = nullptr;
+    void* d_ring = nullptr;
     unsigned grid[2] = {0, 0};  // per direction (different kernels)
     // graph cache
     hipGraphExec_t gexec = nullptr;
@@ -49,8 +54,10 @@ struct UnevenState {
         if (graph) (void)hipGraphDestroy(graph);
         if (cap) (void)hipStreamDestroy(cap);
         if (d_tasks) (void)hipFree(d_tasks);
-        if (d_state) (void)hipFree(d_state);
-        if (d_ws) (void)hipFree(d_ws);
+        if (d_offs) (void)hipFree(d_offs);
+        if (d_init) (void)hipFree(d_init);
+        if (d_ctr) (void)hipFree(d_ctr);
+        if (d_ring) (void)hipFree(d_ring);
     }
 };
 
@@ -61,29 +68,79 @@ static const void* queue_kernel(int isign) {
 
 static int q_cls(int logl, int mode) { return (logl - Q_MIN_LOGL) * Q_MODES + mode; }
 
-// Tasks of one pass over `count` transforms of length L = 2^logl: tiles of TI
-// transforms along b (b-th transform at base + b * bstride), element stride es.
-static void add_pass(std::vector<QTask>& out, int dtype, int logl, int mode, int64_t count, int src, int dst,
-                     int64_t ibase, int64_t ibstride, int32_t iesi, int64_t obase, int64_t obstride, int32_t oeso,
-                     int tw_logn) {
-    const int qp = dtype == NRFFT_F32 ? qpts<float>() : qpts<double>();
-    const int64_t TI = qp >> logl;
-    for (int64_t b0 = 0; b0 < count; b0 += TI) {
+// The two passes of an item: n1a transforms of length 2^la, then n1b = 2^la of
+// length 2^lb = n1a.  First-pass tiles hold ta transforms, second-pass tiles tb.
+struct PassPair {
+    int la, lb;
+    bool cols;  // first pass along columns (four-step), else rows (2-D)
+};
+
+static void add_first(std::vector<QTask>& out, int dtype, const PassPair& p, int64_t off, int64_t ring) {
+    const int64_t pts = dtype == NRFFT_F32 ? fs_tile<float>() : fs_tile<double>();
+    const int64_t LA = int64_t(1) << p.la, LB = int64_t(1) << p.lb, n = LA * LB, cs = (int64_t)csize(dtype);
+    const int64_t ta = std::min(pts / LA, LB), tb = std::min(pts / LB, LA);
+    for (int64_t b0 = 0; b0 < LB; b0 += ta) {
         QTask q{};
-        q.cls = q_cls(logl, mode);
-        q.nvalid = (int32_t)std::min<int64_t>(TI, count - b0);
-        q.src = src;
-        q.dst = dst;
-        q.ioff = ibase + b0 * ibstride;
-        q.ooff = obase + b0 * obstride;
-        q.si0 = (int32_t)ibstride;
-        q.esi = iesi;
-        q.so0 = (int32_t)obstride;
-        q.eso = oeso;
-        q.tw_logn = tw_logn;
-        q.tw_n2base = (int32_t)b0;
+        q.cls = q_cls(p.la, p.cols ? Q_COL : Q_ROWS);
+        q.nvalid = (int32_t)ta;
+        q.ioff = off + (p.cols ? b0 : b0 * LA);
+        q.ibytes = uint32_t((n - (q.ioff - off)) * cs);
+        q.ooff = ring + b0 * tb;
+        q.obytes = uint32_t((n - b0 * tb) * cs);
+        q.ist = (int32_t)(p.cols ? 1 : LA);
+        q.ihi = (int32_t)LB;  // columns
+        q.osh = ilog2((size_t)tb);
+        q.ohi = (int32_t)(LB * tb);
+        q.olo = (int32_t)ta;
+        q.tw_logn = p.la + p.lb;
+        q.first = (int32_t)b0;
         out.push_back(q);
     }
+}
+
+static void add_second(std::vector<QTask>& out, int dtype, const PassPair& p, int64_t off, int64_t ring) {
+    const int64_t pts = dtype == NRFFT_F32 ? fs_tile<float>() : fs_tile<double>();
+    const int64_t LA = int64_t(1) << p.la, LB = int64_t(1) << p.lb, n = LA * LB, cs = (int64_t)csize(dtype);
+    const int64_t ta = std::min(pts / LA, LB), tb = std::min(pts / LB, LA);
+    for (int64_t b0 = 0; b0 < LA; b0 += tb) {
+        QTask q{};
+        q.cls = q_cls(p.lb, Q_RING);
+        q.nvalid = (int32_t)tb;
+        q.ioff = ring + b0 * LB;
+        q.ibytes = uint32_t((n - b0 * LB) * cs);
+        q.ist = (int32_t)ta;
+        q.ish = ilog2((size_t)ta);
+        q.ihi = (int32_t)(tb * ta);
+        q.ooff = off + b0;
+        q.obytes = uint32_t((n - b0) * cs);
+        q.ohi = (int32_t)LA;
+        out.push_back(q);
+    }
+}
+
+// Single-pass items (length, offset; sorted) as tiles of one length: as many
+// items as a tile holds and as its 32-bit offsets reach.
+static std::vector<QTask> single_tiles(int dtype, const std::vector<std::pair<int, int64_t>>& one,
+                                       std::vector<uint32_t>& offs) {
+    std::vector<QTask> out;
+    const int64_t pts = dtype == NRFFT_F32 ? fs_tile<float>() : fs_tile<double>(), cs = (int64_t)csize(dtype);
+    offs.clear();
+    for (size_t i = 0; i < one.size();) {
+        const int logn = one[i].first;
+        const int64_t n = int64_t(1) << logn, base = one[i].second, room = pts >> logn;
+        QTask q{};
+        q.cls = q_cls(logn, Q_ROW);
+        q.ioff = q.ooff = base;
+        q.first = (int32_t)offs.size();
+        for (; i < one.size() && one[i].first == logn && q.nvalid < room; ++i, ++q.nvalid) {
+            const int64_t end = (one[i].second - base + n) * cs;
+            if (end >= int64_t(1) << 31) break;
+            q.ibytes = q.obytes = uint32_t(end);
+            offs.push_back(uint32_t(one[i].second - base));
+        }
+        out.push_back(q);
+    }
+    return out;
 }
 
 // Four-step split of a 1-D item of 2^logn points: the autotuned choice for
@@ -96,57 +153,163 @@ static int uneven_split(int dtype, int logn, int lo, int hi, const std::vector<i
     return std::min(hi, std::max(lo, logn / 2));
 }
 
+// The list of tiles (queue.hpp): items largest first, collected into slabs of
+// at most Q_SLAB_TILES first-pass tiles (or one item) and those into ring slots;
+// second passes stand half a ring behind the first ones; single-pass items are
+// spread evenly over the list, where their arithmetic runs under the others'
+// memory traffic.
 static int build_uneven(UnevenState& u, const std::vector<int>* force_split = nullptr) {
     const bool f32 = u.dtype == NRFFT_F32;
-    const int qlog = ilog2(f32 ? qpts<float>() : qpts<double>());
-    const int maxl = f32 ? q_max_logl<float>() : q_max_logl<double>();
-    // a column tile (TT / JT) holds at least 4 transforms
+    const int qlog = ilog2(f32 ? fs_tile<float>() : fs_tile<double>());
+    const int maxl = std::min(Q_MAX_LOGL, qlog);
+    // a column tile of a four-step holds at least 4 transforms
     const int maxl_col = std::min(maxl, qlog - 2);
-    std::vector<std::pair<int64_t, std::vector<QTask>>> p1, p2;  // (work, tasks) per item
-    size_t ws = 0;
+    struct Two {
+        size_t work;
+        int64_t off;
+        PassPair p;
+    };
+    std::vector<Two> two;
+    std::vector<std::pair<int, int64_t>> one;  // (logn, offset)
     for (const UnevenItem& it : u.items) {
-        std::vector<QTask> a, b;
         if (it.ndim == 1) {
             const int logn = ilog2(it.n0);
             if (logn <= maxl) {
                 if (logn < Q_MIN_LOGL) return fail(NRFFT_E_UNSUPPORTED, "uneven items need N >= 64");
-                add_pass(a, u.dtype, logn, 0, 1, B_IN, B_OUT, it.off, it.n0, 1, it.off, it.n0, 1, 0);
+                one.emplace_back(logn, (int64_t)it.off);
             } else {
                 const int lo = std::max(Q_MIN_LOGL, logn - maxl_col), hi = std::min(maxl_col, logn - Q_MIN_LOGL);
                 if (lo > hi) return fail(NRFFT_E_UNSUPPORTED, "uneven 1-D item longer than the queue supports");
                 const int l1 = uneven_split(u.dtype, logn, lo, hi, force_split);
-                const int l2 = logn - l1;
-                const int64_t N1 = int64_t(1) << l1, N2 = int64_t(1) << l2;
-                // pass A: columns n2 (stride N2), length N1, twiddle -> workspace [k1][n2]
-                add_pass(a, u.dtype, l1, 1, N2, B_IN, B_TMP, (int64_t)it.off, 1, (int32_t)N2, (int64_t)ws, 1,
-                         (int32_t)N2, logn);
-                // pass B: rows k1 of the workspace, length N2, stored at X[k2 N1 + k1]
-                add_pass(b, u.dtype, l2, 2, N1, B_TMP, B_OUT, (int64_t)ws, N2, 1, (int64_t)it.off, 1, (int32_t)N1, 0);
-                ws += size_t(N1 * N2);
+                two.push_back(Two{it.n0, (int64_t)it.off, PassPair{l1, logn - l1, true}});
             }
         } else {
             const int l0 = ilog2(it.n0), l1 = ilog2(it.n1);
             if (l0 < Q_MIN_LOGL || l1 < Q_MIN_LOGL || l1 > maxl || l0 > std::min(maxl, qlog - 1))
                 return fail(NRFFT_E_UNSUPPORTED, "uneven 2-D sides out of the supported range");
-            // rows along n1 (contiguous), then columns along n0 (stride n1) in place in out
-            add_pass(a, u.dtype, l1, 0, (int64_t)it.n0, B_IN, B_OUT, it.off, it.n1, 1, it.off, it.n1, 1, 0);
-            add_pass(b, u.dtype, l0, 1, (int64_t)it.n1, B_OUT, B_OUT, it.off, 1, (int32_t)it.n1, it.off, 1,
-                     (int32_t)it.n1, 0);
+            two.push_back(Two{it.n0 * it.n1, (int64_t)it.off, PassPair{l1, l0, false}});
         }
-        const int64_t work = int64_t(it.n0 * it.n1);
-        p1.emplace_back(work, std::move(a));
-        if (!b.empty()) p2.emplace_back(work, std::move(b));
     }
-    // Largest items first in each phase (longest-processing-time order).
-    auto by_work = [](const auto& x, const auto& y) { return x.first > y.first; };
-    std::stable_sort(p1.begin(), p1.end(), by_work);
-    std::stable_sort(p2.begin(), p2.end(), by_work);
+    std::stable_sort(two.begin(), two.end(), [](const Two& x, const Two& y) { return x.work > y.work; });
+    std::sort(one.begin(), one.end(), [](const auto& x, const auto& y) {
+        return x.first != y.first ? x.first > y.first : x.second < y.second;
+    });
+    const std::vector<QTask> singles = single_tiles(u.dtype, one, u.offs);
+
+    // The ring is handed out front to back, over and over.  Its size is a multiple
+    // of the largest item (and holds at least four), and the items' sizes are powers
+    // of two that do not grow along the list, so no item crosses its end.
+    const size_t largest = two.empty() ? 1 : two[0].work;
+    size_t total = 0;
+    for (const Two& t : two) total += t.work;
+    const size_t ring = std::min(total, std::max<size_t>(4, FUSED_RING_BYTES / csize(u.dtype) / largest) * largest);
+    u.ring_elems = ring;
+    // Slabs: consecutive items.
+    const size_t tile = size_t(1) << qlog, slab_elems = Q_SLAB_TILES * tile;
+    struct Slab {
+        size_t i0, i1, elems, tiles;
+        size_t from;  // ring elements handed out before it; its place is from mod ring
+        int w0, w1;   // slabs [w0, w1) had its place before
+        std::vector<QTask> a, b;
+    };
+    std::vector<Slab> slabs;
+    size_t handed = 0;
+    for (size_t i = 0; i < two.size(); ++i) {
+        const size_t tiles = std::max<size_t>(1, two[i].work / tile);
+        if (slabs.empty() || handed % ring == 0 || slabs.back().elems + two[i].work > slab_elems ||
+            slabs.back().tiles + tiles > Q_SLAB_TILES)
+            slabs.push_back(Slab{i, i, 0, 0, handed, 0, 0, {}, {}});
+        Slab& s = slabs.back();
+        s.i1 = i + 1;
+        s.elems += two[i].work;
+        s.tiles += tiles;
+        handed += two[i].work;
+    }
+    // (A slab's place may begin inside the last one that its predecessor waits for.)
+    for (size_t k = 0, o = 0; k < slabs.size(); ++k) {
+        Slab& s = slabs[k];
+        if (s.from < ring) continue;
+        while (slabs[o].from + slabs[o].elems + ring <= s.from) ++o;
+        s.w0 = (int)o;
+        size_t e = o;
+        while (e < k && slabs[e].from + ring < s.from + s.elems) ++e;
+        s.w1 = (int)e;
+    }
+    u.init.assign(Q_SLABS + 2 * slabs.size(), 0);
+    u.n1 = (int)singles.size();
+    u.n2 = 0;
+    for (size_t k = 0; k < slabs.size(); ++k) {
+        Slab& s = slabs[k];
+        int64_t at = int64_t(s.from % ring);
+        for (size_t i = s.i0; i < s.i1; ++i) {
+            add_first(s.a, u.dtype, two[i].p, two[i].off, at);
+            add_second(s.b, u.dtype, two[i].p, two[i].off, at);
+            at += (int64_t)two[i].work;
+        }
+        const int stored = Q_SLABS + (int)k, loaded = stored + (int)slabs.size();
+        for (QTask& q : s.a) {
+            q.count = stored;
+            q.wait = Q_SLABS + (int)slabs.size() + s.w0;
+            q.nwait = s.w1 - s.w0;
+        }
+        for (QTask& q : s.b) {
+            q.wait = stored;
+            q.nwait = 1;
+            q.count = loaded;
+        }
+        u.init[stored] = (uint32_t)s.a.size();
+        u.init[loaded] = (uint32_t)s.b.size();
+        u.n1 += (int)s.a.size();
+        u.n2 += (int)s.b.size();
+        if (s.w1 - s.w0 > 64) return fail(NRFFT_E_UNSUPPORTED, "uneven ring order");
+    }
+    if ((size_t)u.n1 + (size_t)u.n2 > size_t(1) << 30) return fail(NRFFT_E_UNSUPPORTED, "uneven batch of too many tiles");
+
+    // Few tiles: one group per CU, so that they spread over the chip (720 first-pass
+    // tiles, FP32: 98 us, two per CU 112; 1024: 119 against 108).  If nothing in the
+    // ring is replaced, second passes follow all first ones (925 tiles: 113 us, half
+    // a ring behind 134; 1280: 125 and 136).
+    u.few = (size_t)u.n1 <= Q_FEW_TILES;
+    const size_t lag = ring == total ? ring : ring / 2;
+    // Tickets: a first-pass tile and, once the second passes have begun, one of
+    // theirs, if the distance from a slab's end to its second passes exceeds the
+    // 512 tickets in flight (else second passes wait: 500 items whose largest is
+    // 2048 x 2048, FP32, 680 us against 630); single tiles otherwise.
     u.tasks.clear();
-    for (auto& e : p1) u.tasks.insert(u.tasks.end(), e.second.begin(), e.second.end());
-    u.n1 = (int)u.tasks.size();
-    for (auto& e : p2) u.tasks.insert(u.tasks.end(), e.second.begin(), e.second.end());
-    u.n2 = (int)u.tasks.size() - u.n1;
-    u.ws_elems = ws;
+    u.tasks.reserve(2 * size_t(u.n1 + u.n2));
+    auto ticket = [&](const QTask& x, const QTask* y) {
+        u.tasks.push_back(x);
+        u.tasks.back().last = y == nullptr;
+        u.tasks.push_back(y ? *y : QTask{});
+        u.tasks.back().last = 1;
+    };
+    size_t kb = 0, ib = 0;  // next second-pass tile: slab, index
+    auto second = [&]() -> const QTask* {
+        const QTask* q = &slabs[kb].b[ib];
+        if (++ib == slabs[kb].b.size()) {
+            ib = 0;
+            ++kb;
+        }
+        return q;
+    };
+    size_t done = 0, taken = 0;
+    auto spread = [&](size_t n) {  // n of the two-pass tiles are in the list
+        done += n;
+        const size_t all = size_t(u.n1 + u.n2) - singles.size(), upto = all ? singles.size() * done / all : singles.size();
+        for (; taken < upto; ++taken) ticket(singles[taken], nullptr);
+    };
+    for (const Slab& s : slabs) {
+        for (; (int)kb < s.w1; spread(1)) ticket(*second(), nullptr);
+        for (const QTask& q : s.a) {
+            const bool due = slabs[kb].from + lag <= s.from;
+            const bool pair = due && ring / 2 >= slabs[kb].elems + Q_PAIR_TILES * tile;
+            ticket(q, pair ? second() : nullptr);
+            if (due && !pair) ticket(*second(), nullptr);
+            spread(due ? 2 : 1);
+        }
+    }
+    for (; kb < slabs.size(); spread(1)) ticket(*second(), nullptr);
+    spread(0);
     return NRFFT_OK;
 }
 
@@ -157,19 +320,26 @@ static int uneven_setup_device(UnevenState& u) {
     HIPCHK(hipMalloc(&u.d_tasks, std::max<size_t>(1, u.tasks.size()) * sizeof(QTask)));
     if (!u.tasks.empty())
         HIPCHK(hipMemcpy(u.d_tasks, u.tasks.data(), u.tasks.size() * sizeof(QTask), hipMemcpyHostToDevice));
-    HIPCHK(hipMalloc(&u.d_state, sizeof(QState)));
-    if (u.ws_elems) {
-        const size_t bytes = u.ws_elems * csize(u.dtype);
-        if (hipMalloc(&u.d_ws, bytes) != hipSuccess) return fail(NRFFT_E_NOMEM, "uneven workspace");
+    HIPCHK(hipMalloc(&u.d_offs, std::max<size_t>(1, u.offs.size()) * sizeof(uint32_t)));
+    if (!u.offs.empty())
+        HIPCHK(hipMemcpy(u.d_offs, u.offs.data(), u.offs.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIPCHK(hipMalloc(&u.d_init, u.init.size() * sizeof(uint32_t)));
+    HIPCHK(hipMemcpy(u.d_init, u.init.data(), u.init.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    std::vector<uint32_t> ctr(u.init.size() * Q_LINE, 0);
+    for (size_t i = 0; i < u.init.size(); ++i) ctr[i * Q_LINE] = u.init[i];
+    HIPCHK(hipMalloc(&u.d_ctr, ctr.size() * sizeof(uint32_t)));
+    HIPCHK(hipMemcpy(u.d_ctr, ctr.data(), ctr.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    if (u.ring_elems) {
+        const size_t bytes = u.ring_elems * csize(u.dtype);
+        if (hipMalloc(&u.d_ring, bytes) != hipSuccess) return fail(NRFFT_E_NOMEM, "uneven workspace");
     }
     for (int d = 0; d < 2; ++d) {
         const void* fn = u.dtype == NRFFT_F32 ? queue_kernel<float>(d == 0 ? 1 : -1)
                                               : queue_kernel<double>(d == 0 ? 1 : -1);
-        const int nt = u.dtype == NRFFT_F32 ? qpts<float>() / 16 : qpts<double>() / 16;
         int per_cu = 0;
-        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, nt, 0));
+        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, FS_NT, 0));
         if (per_cu < 1) return fail(NRFFT_E_UNSUPPORTED, "queue kernel does not fit a CU");
-        u.grid[d] = (unsigned)(per_cu * ctx->ncu);
+        u.grid[d] = (unsigned)((u.few ? 1 : per_cu) * ctx->ncu);
     }
     HIPCHK(hipStreamCreateWithFlags(&u.cap, hipStreamNonBlocking));
     return NRFFT_OK;
@@ -181,22 +351,18 @@ static int uneven_enqueue(UnevenState& u, const void* in, void* out, int isign, 
     int rc = get_ctx(&ctx);
     if (rc) return rc;
     Twiddles<T> tw = ctx_twiddles<T>(ctx);
-    cpx<T>* pin = const_cast<cpx<T>*>(static_cast<const cpx<T>*>(in));
+    const cpx<T>* pin = static_cast<const cpx<T>*>(in);
     cpx<T>* pout = static_cast<cpx<T>*>(out);
-    cpx<T>* pws = static_cast<cpx<T>*>(u.d_ws);
+    cpx<T>* ring = static_cast<cpx<T>*>(u.d_ring);
     const QTask* tk = u.d_tasks;
-    QState* st = u.d_state;
-    const int d = isign > 0 ? 0 : 1;
-    hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, s, st);
-    HIPCHK(hipGetLastError());
-    const int nt = (int)(qpts<T>() / 16);
-    for (int phase = 0; phase < 2; ++phase) {
-        int base = phase ? u.n1 : 0, count = phase ? u.n2 : u.n1, ph = phase;
-        if (count == 0) continue;
-        const unsigned grid = std::min<unsigned>(u.grid[d], (unsigned)count);
-        void* args[] = {&pin, &pout, &pws, &tk, &base, &count, &ph, &st, &tw};
-        HIPCHK(hipLaunchKernel(queue_kernel<T>(isign), dim3(grid), dim3(nt), args, 0, s));
-    }
+    uint32_t* ctr = u.d_ctr;
+    const uint32_t* init = u.d_init;
+    int lines = (int)u.init.size();
+    const uint32_t* offs = u.d_offs;
+    int count = (int)u.tasks.size();
+    const unsigned grid = std::min<unsigned>(u.grid[isign > 0 ? 0 : 1], unsigned(count / 2));
+    void* args[] = {&pin, &pout, &ring, &tk, &count, &offs, &ctr, &init, &lines, &tw};
+    HIPCHK(hipLaunchKernel(queue_kernel<T>(isign), dim3(grid), dim3(FS_NT), args, 0, s));
     return NRFFT_OK;
 }
 
@@ -256,8 +422,8 @@ static int time_uneven(UnevenState& u, void* in, void* out, int iters, hipStream
 // tune cache under (PK_UNEVEN, dtype, {N}).
 static int autotune_uneven(int dtype, int lmin, int lmax, int iters, int* best_l1, float* best_ms) {
     const bool f32 = dtype == NRFFT_F32;
-    const int qlog = ilog2(f32 ? qpts<float>() : qpts<double>());
-    const int maxl = f32 ? q_max_logl<float>() : q_max_logl<double>();
+    const int qlog = ilog2(f32 ? fs_tile<float>() : fs_tile<double>());
+    const int maxl = std::min(Q_MAX_LOGL, qlog);
     const int maxl_col = std::min(maxl, qlog - 2);
     const size_t pts = size_t(1) << (f32 ? 25 : 24);
     struct Res {
@@ -433,12 +599,12 @@ int nrfft_execute_uneven_nograph(nrfft_uneven plan, const void* d_in, void* d_ou
 int nrfft_uneven_check(nrfft_uneven plan, void* stream) {
     g_err.clear();
     if (!plan) return fail(NRFFT_E_INVALID, "null plan");
-    QState st{};
-    HIPCHK(hipMemcpyAsync(&st, plan->u.d_state, sizeof st, hipMemcpyDeviceToHost, (hipStream_t)stream));
+    uint32_t tickets = 0;
+    HIPCHK(hipMemcpyAsync(&tickets, plan->u.d_ctr + Q_LAST * Q_LINE, sizeof tickets, hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
-    // every group leaves after drawing one index past the end of its phase
-    if (st.next[0] < (uint32_t)plan->u.n1 || st.next[1] < (uint32_t)plan->u.n2)
-        return fail(NRFFT_E_HIP, "uneven queue: a phase did not drain its task list");
+    // every group leaves after drawing one ticket past the end
+    if (2 * (uint64_t)tickets < (uint64_t)plan->u.tasks.size())
+        return fail(NRFFT_E_HIP, "uneven queue: the task list was not drained");
     return NRFFT_OK;
 }
 
@@ -448,7 +614,7 @@ int nrfft_uneven_info(nrfft_uneven plan, size_t* tasks_phase1, size_t* tasks_pha
     if (!plan) return fail(NRFFT_E_INVALID, "null plan");
     if (tasks_phase1) *tasks_phase1 = (size_t)plan->u.n1;
     if (tasks_phase2) *tasks_phase2 = (size_t)plan->u.n2;
-    if (workspace_bytes) *workspace_bytes = plan->u.ws_elems * csize(plan->u.dtype);
+    if (workspace_bytes) *workspace_bytes = plan->u.ring_elems * csize(plan->u.dtype);
     if (groups) *groups = plan->u.grid[0];
     return NRFFT_OK;
 }

@@ -336,7 +336,7 @@ class UnevenPlan(_Plan):
 
     @property
     def num_launches(self) -> int:
-        return 3  # counter reset, phase 1, phase 2
+        return 1
 
     def execute(self, x_in, x_out, isign: int, stream=None, graph: bool = True) -> None:
         fn = _lib.lib().nrfft_execute_uneven if graph else _lib.lib().nrfft_execute_uneven_nograph
