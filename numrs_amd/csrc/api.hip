@@ -419,16 +419,16 @@ int plan_c2c_1d(Plan& p, int logn, int64_t batch, int src, int dst, size_t* tmp_
 // tuning only: an explicit or cached tuning names the split, tiles and chunk
 // of separate passes.
 bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* out,
-                  size_t* ring_elems) {
+                  size_t* ring_elems, bool real) {
     if (p.kind == PK_C2C && p.extra != 0) return false;
     const size_t n = size_t(1) << logn;
     if (!(p.tune == default_tune_1d(p.dtype, n, p.batch, 0))) return false;
     const bool f32 = p.dtype == NRFFT_F32;
-    const FusedRef fp = f32 ? fused_lookup_f32(1, logn) : fused_lookup_f64(1, logn);
-    const FusedRef fm = f32 ? fused_lookup_f32(-1, logn) : fused_lookup_f64(-1, logn);
+    const FusedRef fp = f32 ? fused_lookup_f32(1, logn, real) : fused_lookup_f64(1, logn, real);
+    const FusedRef fm = f32 ? fused_lookup_f32(-1, logn, real) : fused_lookup_f64(-1, logn, real);
     if (!fp.fn || !fm.fn) return false;
     const int64_t tiles = batch << fp.tiles_log;
-    if (tiles < fused_min_tiles(f32, logn) || tiles >= (int64_t(1) << 30)) return false;
+    if (tiles < fused_min_tiles(f32, logn, real) || tiles >= (int64_t(1) << 30)) return false;
     DeviceCtx* ctx = nullptr;
     if (get_ctx(&ctx)) return false;
     int per_cu = 0;

@@ -42,6 +42,7 @@
 // the very last group finds the others gone and clears everything.)
 #pragma once
 #include "pass_c2c.hpp"
+#include "real_fft.hpp"
 
 namespace nrfft {
 
@@ -172,8 +173,16 @@ struct FsLtw {
 //   MAPS = MAP_J  contiguous ([t][L]), a gap of one after every LANES values.
 // Reads and the later exchanges' writes take (nearly) consecutive addresses.
 // ---------------------------------------------------------------------------
-template <typename T, int S, int L, int MAPL, int MAPS = MAP_T>
+//
+// PAIR = FS_PAIR_FIRST / FS_PAIR_LAST: the values of the first (last) stage are
+// held in mirror pairs.  Lane l + 32 of a wave then has butterfly NB - 1 - j of
+// transform t + TI / 2 where lane l has butterfly j of transform t < TI / 2, so
+// element i of one and L - 1 - i of the other stand in registers r and R - 1 - r.
+enum { FS_PAIR_FIRST = 1, FS_PAIR_LAST = 2 };
+template <typename T, int S, int L, int MAPL, int MAPS = MAP_T, int PAIR = 0>
 struct FsEng {
+    static_assert(!(PAIR & FS_PAIR_FIRST) || MAPL == MAP_T, "pairs lie across the transforms");
+    static_assert(!(PAIR & FS_PAIR_LAST) || MAPS == MAP_T, "pairs lie across the transforms");
     static_assert(MAPS == MAP_T || MAPL == MAP_J, "row stores come with row loads");
     using P = FsPlan<T, L>;
     static constexpr int EPT = fs_ept<T>(), NT = FS_NT, TI = fs_tile<T>() / L, NST = P::NST;
@@ -210,7 +219,13 @@ struct FsEng {
         for (int b = 0; b < BPT; ++b) {
             const unsigned q = unsigned(tid) + unsigned(b * NT);
             int t, j;
-            if constexpr ((s == 0 ? MAPL : MAPS) == MAP_J) {
+            if constexpr ((s == 0 && (PAIR & FS_PAIR_FIRST)) || (s == NST - 1 && (PAIR & FS_PAIR_LAST))) {
+                const unsigned ql = unsigned(tid / 64 * 32 + tid % 32) + unsigned(b * (NT / 2)), jj = ql / unsigned(TI / 2);
+                const bool up = (tid & 32) != 0;
+                j = (s == 0 && G > 1) ? int((jj % unsigned(G)) * unsigned(NB / G) + jj / unsigned(G)) : int(jj);
+                t = int(ql % unsigned(TI / 2)) + (up ? TI / 2 : 0);
+                j = up ? NB - 1 - j : j;
+            } else if constexpr ((s == 0 ? MAPL : MAPS) == MAP_J) {
                 t = int(q / unsigned(NB));
                 j = int(q % unsigned(NB));
             } else {
@@ -399,6 +414,69 @@ __device__ __forceinline__ void fs_count(uint32_t* p) {
     __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ---------------------------------------------------------------------------
+// The untangle of a real transform (untangle_pair, real_fft.hpp) on mirror pairs
+// in registers: bins p and N - p of the packed signal stand in registers r and
+// R - 1 - r of a thread and of the one 32 lanes away (FS_PAIR_*).
+// ---------------------------------------------------------------------------
+// exp(i pi r / R), r < R <= 32.
+template <int R, int r, typename T>
+__device__ __forceinline__ cpx<T> fs_half_root() {
+    constexpr double c[17] = {1.0, 0.99518472667219688624483695310948, 0.98078528040323044912618223613424,
+                              0.95694033573220886493579788698027, 0.92387953251128675612818318939679,
+                              0.88192126434835502971275686366039, 0.83146961230254523707878837761791,
+                              0.77301045336273696081090660975847, 0.70710678118654752440084436210485,
+                              0.63439328416364549821517161322549, 0.55557023301960222474283081394853,
+                              0.47139673682599764855638762590525, 0.38268343236508977172845998403040,
+                              0.29028467725446236763619237581740, 0.19509032201612826784828486847702,
+                              0.09801714032956060199419556388864, 0.0};
+    constexpr int k = r * (32 / R);
+    constexpr double re = k <= 16 ? c[k <= 16 ? k : 0] : -c[k <= 16 ? 0 : 32 - k];
+    constexpr double im = c[k <= 16 ? 16 - k : k - 16];
+    return {(T)re, (T)im};
+}
+// The value of the lane 32 away.
+__device__ __forceinline__ float fs_cross(float x, bool up) {
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // {low half twice, high half twice}
+    return __builtin_bit_cast(float, up ? r[0] : r[1]);
+}
+__device__ __forceinline__ double fs_cross(double x, bool up) {
+    const auto u = __builtin_bit_cast(fs_u2, x);
+    const auto a = __builtin_amdgcn_permlane32_swap(u[0], u[0], false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(u[1], u[1], false, false);
+    return __builtin_bit_cast(double, fs_u2{up ? a[0] : a[1], up ? b[0] : b[1]});
+}
+template <typename T>
+__device__ __forceinline__ cpx<T> fs_cross(cpx<T> v, bool up) {
+    return {fs_cross(v.x, up), fs_cross(v.y, up)};
+}
+// Butterfly of R values at v, w0 = exp(i pi p / N) of its bin r = 0 (DIR = -1:
+// the conjugate).  v[R - 1 - r] becomes the mirror of v[r]'s bin, r < R / 2.
+template <int DIR, int R, int r = 0, typename T>
+__device__ __forceinline__ void fs_untangle(cpx<T>* v, cpx<T> w0, bool up) {
+    if constexpr (r < R / 2) {
+        const cpx<T> w = cmul(w0, dirw<DIR>(fs_half_root<R, r, T>()));
+        cpx<T> x, y;
+        untangle_pair(v[r], fs_cross(v[R - 1 - r], up), w, (T)(-0.5 * DIR), x, y);
+        v[r] = x;
+        v[R - 1 - r] = y;
+        fs_untangle<DIR, R, r + 1>(v, w0, up);
+    }
+}
+// Likewise of a transform that is its own mirror, partner(r) = the value at the
+// mirror of bin r: v[r] stays bin r.  dc: v[0] is bin 0.
+template <int DIR, int R, int r = 0, typename T, class P>
+__device__ __forceinline__ void fs_untangle_self(cpx<T>* v, cpx<T> w0, bool dc, P&& partner) {
+    if constexpr (r < R) {
+        const cpx<T> w = cmul(w0, dirw<DIR>(fs_half_root<R, r, T>()));
+        cpx<T> x, y;
+        untangle_pair(v[r], partner(r), w, (T)(-0.5 * DIR), x, y);
+        v[r] = r == 0 && dc ? (DIR > 0 ? dc_forward(v[r]) : dc_inverse(v[r])) : x;
+        fs_untangle_self<DIR, R, r + 1>(v, w0, dc, partner);
+    }
+}
+
 template <typename T, int LA, int LB>
 struct FsShape {
     static constexpr int TILE = fs_tile<T>();
@@ -423,12 +501,25 @@ struct FsShape {
 // CU's two groups the one further along finishes first (oldest-first issue let
 // the younger group's A tiles take 30 us beside 14, and every slab waits for
 // its slowest tile: 311 -> 302 us with a lag of 8 slabs, zero data).
-template <typename T, int S, int LA, int LB>
+//
+// RE = 1: the forward transform of 2 N reals (S = 1), RE = -1: its inverse (S =
+// -1); N and the tables are those of the packed signal.  Bin p = k2 LA + k1 pairs
+// with N - p in row LA - k1 (row 0 with itself, row LA / 2 too), so a pass-B tile of
+// RE = 1 holds TB / 2 rows k1 = c .. and their mirror rows, taken from the ring
+// where they lie; the rows 0 and LA / 2 share a pair's place and are untangled
+// through the LDS.  RE = -1 takes column tiles likewise (columns n2 and LB - n2),
+// untangles before pass A, and pass B picks the columns up in their order.  So the
+// untangle costs no pass over memory.  64 x 2^19 reals FP32 (the data of 32 x 2^19
+// complex) forward 160 us, inverse 163, in passes 313 and 255; 37 x 2^20 134 and
+// 117 against 195 and 134.  What it pays instead: half as long runs in memory, one
+// of two at an odd element.
+template <typename T, int S, int LA, int LB, int RE = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(FS_NT, FS_NT), amdgpu_waves_per_eu(4, 4))) void
 k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twiddles<T> tw) {
+    static_assert(RE == 0 || RE == S, "forward untangles behind, the inverse ahead");
     using SH = FsShape<T, LA, LB>;
-    using EA = FsEng<T, S, LA, MAP_T>;
-    using EB = FsEng<T, S, LB, MAP_J>;
+    using EA = FsEng<T, S, LA, MAP_T, MAP_T, (RE < 0 ? FS_PAIR_FIRST : 0)>;
+    using EB = FsEng<T, S, LB, MAP_J, MAP_T, (RE > 0 ? FS_PAIR_LAST : 0)>;
     constexpr int TILE = SH::TILE, TA = SH::TA, TB = SH::TB, EPT = fs_ept<T>(), CS = (int)sizeof(cpx<T>);
     constexpr int TPT_LOG = ilog2c(SH::NTA);  // tiles per transform
     constexpr int64_t N = SH::N;
@@ -543,15 +634,61 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                 fs_count(pending);
             }
         };
+        // Column (RE < 0) or row (RE > 0) tt of the tile.
+        auto paired = [&](int tt, int half, int len) {
+            const uint32_t u = idx * uint32_t(half) + uint32_t(tt & (half - 1));
+            return tt < half ? u : u ? uint32_t(len) - u : uint32_t(len / 2);
+        };
+        auto column = [&](int tt) {
+            if constexpr (RE < 0) return paired(tt, TA / 2, LB);
+            else return idx * uint32_t(TA) + uint32_t(tt);
+        };
+        // Untangle of the tile's mirror pairs, transforms of
+        // length L in butterflies of radix R: each(f) goes through the butterflies, bin(t, j) is the bin of
+        // a butterfly's first value; back: the mirrors return to their threads.
+        auto untangle = [&](auto radix, auto len, cpx<T>* x, int id, auto&& each, auto&& bin, bool back) {
+            constexpr int R = decltype(radix)::value, L = decltype(len)::value, NB = L / R;
+            const bool up = (id & 32) != 0;
+            constexpr int HALF = TILE / L / 2;
+            auto own = [&](int tt) { return idx == 0 && (tt & (HALF - 1)) == 0; };
+            if (idx == 0) {  // transforms that are their own mirrors
+                cpx<T>* z = reinterpret_cast<cpx<T>*>(ex) + (up ? L : 0);
+                lds_barrier();
+                each([&](int b, int tt, int j) {
+                    if (own(tt))
+#pragma unroll
+                        for (int r = 0; r < R; ++r) z[j + r * NB] = x[b * R + r];
+                });
+                lds_barrier();
+                each([&](int b, int tt, int j) {
+                    if (own(tt))
+                        fs_untangle_self<RE, R>(x + b * R, twiddle_big<RE>(tw, bin(tt, j), LOGN + 1), j == 0 && !up,
+                                                [&](int r) {
+                                                    const int k = j + r * NB;
+                                                    return z[up ? L - 1 - k : (L - k) & (L - 1)];
+                                                });
+                });
+                lds_barrier();
+            }
+            each([&](int b, int tt, int j) {
+                if (!own(tt)) {
+                    fs_untangle<RE, R>(x + b * R, twiddle_big<RE>(tw, bin(tt, j), LOGN + 1), up);
+                    if (back)
+#pragma unroll
+                        for (int r = R / 2; r < R; ++r) x[b * R + r] = fs_cross(x[b * R + r], up);
+                }
+            });
+        };
         if (!t.b) {
             const __amdgpu_buffer_rsrc_t rin = fs_rsrc(in + int64_t(tr) * N, uint32_t(N * CS));
             // x[(j + r NB0) LB + idx TA + t]
             EA::template each_butterfly<0>(ltid, [&](int b, int tt, int j) {
                 constexpr int R = EA::R0, NB = LA / R;
-                const uint32_t voff = uint32_t(j * LB + tt) * CS;
+                const uint32_t voff = uint32_t(j * LB) * CS + (RE < 0 ? column(tt) * uint32_t(CS) : uint32_t(tt * CS));
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    v[b * R + r] = fs_load<T, FS_AUX_NT>(rin, voff, uint32_t(r * NB * LB) * CS + idx * uint32_t(TA * CS));
+                    v[b * R + r] = fs_load<T, FS_AUX_NT>(
+                        rin, voff, uint32_t(r * NB * LB) * CS + (RE < 0 ? 0u : idx * uint32_t(TA * CS)));
             });
             publish();
             if (last_of_unit(k)) take_ticket();
@@ -559,12 +696,18 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             auto load_tw = [&]() {
                 uint32_t n2 = 0, jl[EPT / EA::RL];
                 EA::template each_butterfly<EA::NST - 1>(ltid, [&](int b, int tt, int j) {
-                    n2 = idx * uint32_t(TA) + uint32_t(tt);  // the same for every b
+                    n2 = column(tt);  // the same for every b
                     jl[b] = uint32_t(j);
                 });
                 f.load(tw, n2, jl, LOGN);
             };
             __builtin_amdgcn_s_setprio(1);
+            if constexpr (RE < 0) {
+                untangle(
+                    std::integral_constant<int, EA::R0>{}, std::integral_constant<int, LA>{}, v, ltid,
+                    [&](auto&& f) { EA::template each_butterfly<0>(ltid, f); },
+                    [&](int tt, int j) { return uint32_t(j * LB) + column(tt); }, true);
+            }
             EA::template butterflies<0>(v);
             EA::rest(
                 v, ltid, ex, typename EA::Ltw{ltwa}, tw.stage, load_tw,
@@ -592,16 +735,47 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             __builtin_amdgcn_s_setprio(0);
             pending = st->stored[t.slot];
         } else {
-            const __amdgpu_buffer_rsrc_t rr = fs_rsrc(rt + int64_t(idx) * TILE, uint32_t(TILE * CS));
-            // row t, element i: (i / TA) TB TA + t TA + i mod TA
+            // row t, element i: (i / TA) TB TA + t TA + i mod TA from its tile
+            const __amdgpu_buffer_rsrc_t rr =
+                RE > 0 ? fs_rsrc(rt, uint32_t(N * CS)) : fs_rsrc(rt + int64_t(idx) * TILE, uint32_t(TILE * CS));
             EB::template each_butterfly<0>(ltid, [&](int b, int tt, int j) {
-                constexpr int R = EB::R0, NB = LB / R;
+                constexpr int R = EB::R0, NB = LB / R, H = TA / 2;
                 static_assert(NB % TA == 0 || TA % NB == 0, "input steps are constant");
-                const uint32_t voff = uint32_t((j / TA) * (TB * TA) + tt * TA + j % TA) * CS;
+                uint32_t row = uint32_t(tt * TA);
+                if constexpr (RE > 0) {
+                    const uint32_t k1 = paired(tt, TB / 2, LA);
+                    row = (k1 / TB) * uint32_t(TILE) + (k1 % TB) * uint32_t(TA);
+                }
+                if constexpr (RE < 0) {
+                    // column n2 < LB / 2 is column n2 mod H of tile n2 / H, its mirror LB - n2 (column
+                    // 0: LB / 2) the one H further on
+                    auto at = [&](uint32_t n) { return (n / H) * uint32_t(TB * TA) + n % H; };
 #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    v[b * R + r] = fs_load<T, FS_AUX_SC1>(
-                        rr, voff, uint32_t(((r * NB) / TA) * (TB * TA) + (r * NB) % TA) * CS);
+                    for (int r = 0; r < R; ++r) {
+                        uint32_t voff, soff;
+                        if constexpr (NB % H == 0) {  // steps are constant
+                            if (r < R / 2) {
+                                voff = at(uint32_t(j));
+                                soff = uint32_t((r * NB) / H * (TB * TA));
+                            } else {
+                                voff = at(uint32_t(NB - j)) + H;
+                                soff = uint32_t(((R - 1 - r) * NB) / H * (TB * TA));
+                                if (r == R / 2 && j == 0) voff = H - soff;
+                            }
+                        } else {
+                            const uint32_t n2 = uint32_t(j + r * NB);
+                            voff = n2 < uint32_t(LB / 2) ? at(n2) : at(n2 == LB / 2 ? 0u : uint32_t(LB) - n2) + H;
+                            soff = 0;
+                        }
+                        v[b * R + r] = fs_load<T, FS_AUX_SC1>(rr, (voff + soff + row) * uint32_t(CS), 0);
+                    }
+                } else {
+                    const uint32_t voff = ((j / TA) * uint32_t(TB * TA) + row + uint32_t(j % TA)) * uint32_t(CS);
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        v[b * R + r] = fs_load<T, FS_AUX_SC1>(
+                            rr, voff, uint32_t(((r * NB) / TA) * (TB * TA) + (r * NB) % TA) * CS);
+                }
             });
             publish();
             if (last_of_unit(k)) take_ticket();
@@ -619,12 +793,25 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                     __builtin_amdgcn_s_setprio(3);
                 });
             const __amdgpu_buffer_rsrc_t ro = fs_rsrc(out + int64_t(tr) * N, uint32_t(N * CS));
+            if constexpr (RE > 0)
+                untangle(
+                    std::integral_constant<int, EB::RL>{}, std::integral_constant<int, LB>{}, v, ltid,
+                    [&](auto&& f) { EB::template each_butterfly<EB::NST - 1>(ltid, f); },
+                    [&](int tt, int j) { return uint32_t(j * LA) + paired(tt, TB / 2, LA); }, false);
             EB::template each_butterfly<EB::NST - 1>(ltid, [&](int b, int tt, int j) {
                 constexpr int R = EB::RL, NB = EB::NBL;
-                const uint32_t voff = uint32_t(j * LA + tt) * CS;
+                uint32_t voff = uint32_t(j * LA + tt) * CS, mirror = voff;
+                if constexpr (RE > 0) {
+                    const uint32_t k1 = paired(tt, TB / 2, LA);
+                    voff = (uint32_t(j * LA) + k1) * uint32_t(CS);
+                    mirror = idx == 0 && (tt & (TB / 2 - 1)) == 0
+                                 ? voff
+                                 : (uint32_t((NB - 1 - j) * LA) + uint32_t(LA) - k1) * uint32_t(CS);
+                }
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    fs_store<T, FS_AUX_NT>(v[b * R + r], ro, voff, uint32_t(r * NB * LA) * CS + idx * uint32_t(TB * CS));
+                    fs_store<T, FS_AUX_NT>(v[b * R + r], ro, r < R / 2 ? voff : mirror,
+                                           uint32_t(r * NB * LA) * CS + (RE > 0 ? 0u : idx * uint32_t(TB * CS)));
             });
             __builtin_amdgcn_s_setprio(0);
             pending = nullptr;

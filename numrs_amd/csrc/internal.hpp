@@ -211,19 +211,24 @@ struct FusedRef {
     const void* fn;
     int tiles_log;  // log2 tiles of one pass per transform
 };
-FusedRef fused_lookup_f32(int sign, int logn);
-FusedRef fused_lookup_f64(int sign, int logn);
+// real: the forward / inverse transform of 2^(logn + 1) reals.
+FusedRef fused_lookup_f32(int sign, int logn, bool real);
+FusedRef fused_lookup_f64(int sign, int logn, bool real);
 // The fused launch of `batch` transforms of 2^logn points from src to dst
 // with a ring of at most ring_bytes; false if the size has no such kernel or
 // runs faster as separate passes.  *ring_elems: complex values of its ring.
 bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* l,
-                  size_t* ring_elems);
+                  size_t* ring_elems, bool real = false);
 // Fewest tiles of a pass for the fused launch (its lead-in and its tail run
 // one pass only).  MI355X, buffers changing from call to call, fused against
 // separate passes: FP32 2^20 640 tiles 68.7 / 74.9 us, 512 tiles 58.7 / 60.1,
 // 384 tiles 52.1 / 47.8; FP32 2^15 640 tiles 66.7 / 67.2; FP64 2^16 640 tiles
-// 63.7 / 68.3; FP64 2^18 768 tiles 74.9 / 75.9, 640 tiles 67.2 / 64.1.
-inline int64_t fused_min_tiles(bool f32, int logn) { return !f32 && logn >= 18 ? 1024 : 640; }
+// 63.7 / 68.3; FP64 2^18 768 tiles 74.9 / 75.9, 640 tiles 67.2 / 64.1.  Real, both
+// directions: FP32 2^19 640 tiles 167 / 170 us; 2^20 640 tiles 201 / 196, 1184 317 /
+// 392; 2^21 640 tiles 227 / 204, 1184 361 / 392.
+inline int64_t fused_min_tiles(bool f32, int logn, bool real) {
+    return (f32 ? real && logn >= 20 : logn >= 18) ? 1024 : 640;
+}
 constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;
 bool plan_is_fused(const Plan& p);
 // A zeroed FsState of the current device's pool for a plan with fused
