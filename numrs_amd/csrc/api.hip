@@ -419,16 +419,16 @@ int plan_c2c_1d(Plan& p, int logn, int64_t batch, int src, int dst, size_t* tmp_
 // tuning only: an explicit or cached tuning names the split, tiles and chunk
 // of separate passes.
 bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* out,
-                  size_t* ring_elems, bool real) {
+                  size_t* ring_elems, int form, int64_t least_tiles) {
     if (p.kind == PK_C2C && p.extra != 0) return false;
     const size_t n = size_t(1) << logn;
     if (!(p.tune == default_tune_1d(p.dtype, n, p.batch, 0))) return false;
     const bool f32 = p.dtype == NRFFT_F32;
-    const FusedRef fp = f32 ? fused_lookup_f32(1, logn, real) : fused_lookup_f64(1, logn, real);
-    const FusedRef fm = f32 ? fused_lookup_f32(-1, logn, real) : fused_lookup_f64(-1, logn, real);
+    const FusedRef fp = f32 ? fused_lookup_f32(1, logn, form) : fused_lookup_f64(1, logn, form);
+    const FusedRef fm = f32 ? fused_lookup_f32(-1, logn, form) : fused_lookup_f64(-1, logn, form);
     if (!fp.fn || !fm.fn) return false;
     const int64_t tiles = batch << fp.tiles_log;
-    if (tiles < fused_min_tiles(f32, logn, real) || tiles >= (int64_t(1) << 30)) return false;
+    if (tiles < (least_tiles ? least_tiles : fused_min_tiles(f32, logn, form)) || tiles >= (int64_t(1) << 30)) return false;
     DeviceCtx* ctx = nullptr;
     if (get_ctx(&ctx)) return false;
     int per_cu = 0;
@@ -441,11 +441,11 @@ bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size
     l.kind = LK_FUSED;
     l.fn[0] = fp.fn;
     l.fn[1] = fm.fn;
-    l.src = src;
-    l.dst = dst;
+    l.src = l.src2 = src;
+    l.dst = l.dst2 = dst;
     l.nt = FS_NT;
     l.grid = (unsigned)std::min<int64_t>(2 * tiles, int64_t(per_cu) * ctx->ncu);
-    l.fs.batch = (int32_t)batch;
+    l.fs.batch = l.fs.split = (int32_t)batch;
     l.fs.slab_log = std::max(0, 6 - fp.tiles_log);
     const int64_t slabs = (batch + (int64_t(1) << l.fs.slab_log) - 1) >> l.fs.slab_log;
     const size_t slab_elems = n << l.fs.slab_log;
@@ -807,15 +807,38 @@ int exec_launch(const Plan& p, const Launch& l, void* const* bufs, int isign, hi
         void* ring = bufs[B_TMP];
         void* state = bufs[B_STATE];
         if (!ring || !state) return fail(NRFFT_E_INVALID, "fused launch without its workspace");
-        if (p.dtype == NRFFT_F32) {
-            Twiddles<float> tw = ctx_twiddles<float>(ctx);
-            void* args[] = {&a, &b, &ring, &state, &d, &tw};
-            HIPCHK(hipLaunchKernel(l.fn[si], dim3(l.grid), dim3(l.nt), args, 0, stream));
-        } else {
-            Twiddles<double> tw = ctx_twiddles<double>(ctx);
-            void* args[] = {&a, &b, &ring, &state, &d, &tw};
-            HIPCHK(hipLaunchKernel(l.fn[si], dim3(l.grid), dim3(l.nt), args, 0, stream));
+        void* a2 = bufs[l.src2];
+        void* b2 = bufs[l.dst2];
+        auto launch = [&]() {
+            Twiddles<float> tf;
+            Twiddles<double> td;
+            void* args[] = {&a, &b, &ring, &state, &d, nullptr, &a2, &b2};
+            if (p.dtype == NRFFT_F32) {
+                tf = ctx_twiddles<float>(ctx);
+                args[5] = &tf;
+            } else {
+                td = ctx_twiddles<double>(ctx);
+                args[5] = &td;
+            }
+            return hipLaunchKernel(l.fn[si], dim3(l.grid), dim3(l.nt), args, 0, stream);
+        };
+        if (d.split < d.batch) {
+            // The first transforms' outputs are stored while the second inputs
+            // are still read: if they overlap, one after the other, these first.
+            const size_t per = p.nn[0] / 2 * csize(p.dtype);
+            const char *o = static_cast<char*>(b), *i = static_cast<char*>(a2);
+            if (o < i + per * size_t(d.batch - d.split) && i < o + per * size_t(d.split)) {
+                std::swap(a, a2);
+                std::swap(b, b2);
+                const int32_t n0 = d.split, n1 = d.batch - d.split;
+                d.batch = d.split = n1;
+                HIPCHK(launch());
+                std::swap(a, a2);
+                std::swap(b, b2);
+                d.batch = d.split = n0;
+            }
         }
+        HIPCHK(launch());
         return NRFFT_OK;
     }
     if (l.kind == LK_C2C) {

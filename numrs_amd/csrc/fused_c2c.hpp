@@ -61,6 +61,7 @@ struct FsState {
 
 struct FsDesc {
     int32_t batch;       // transforms
+    int32_t split;       // transforms of `in` and `out`; the others are those of `in2` and `out2`
     int32_t slab_log;    // log2 transforms per slab
     int32_t slots;       // ring slots (slabs)
     int32_t lag;         // slabs pass B trails pass A by, 1 .. slots - 1
@@ -513,10 +514,15 @@ struct FsShape {
 // complex) forward 160 us, inverse 163, in passes 313 and 255; 37 x 2^20 134 and
 // 117 against 195 and 134.  What it pays instead: half as long runs in memory, one
 // of two at an odd element.
+//
+// RE = -2: the inverse of the correlation of the spectra `in` and `in2`: as RE = -1
+// on a conj(b) / N, taken where a tile is loaded (b in pieces of 8 values a thread;
+// more would not fit beside a).
 template <typename T, int S, int LA, int LB, int RE = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(FS_NT, FS_NT), amdgpu_waves_per_eu(4, 4))) void
-k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twiddles<T> tw) {
-    static_assert(RE == 0 || RE == S, "forward untangles behind, the inverse ahead");
+k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twiddles<T> tw, const cpx<T>* in2,
+         cpx<T>* out2) {
+    static_assert(RE == 0 || (RE > 0) == (S > 0), "forward untangles behind, the inverse ahead");
     using SH = FsShape<T, LA, LB>;
     using EA = FsEng<T, S, LA, MAP_T, MAP_T, (RE < 0 ? FS_PAIR_FIRST : 0)>;
     using EB = FsEng<T, S, LB, MAP_J, MAP_T, (RE > 0 ? FS_PAIR_LAST : 0)>;
@@ -639,7 +645,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             const uint32_t u = idx * uint32_t(half) + uint32_t(tt & (half - 1));
             return tt < half ? u : u ? uint32_t(len) - u : uint32_t(len / 2);
         };
-        auto column = [&](int tt) {
+        auto column = [&](int tt) -> uint32_t {
             if constexpr (RE < 0) return paired(tt, TA / 2, LB);
             else return idx * uint32_t(TA) + uint32_t(tt);
         };
@@ -662,7 +668,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                 lds_barrier();
                 each([&](int b, int tt, int j) {
                     if (own(tt))
-                        fs_untangle_self<RE, R>(x + b * R, twiddle_big<RE>(tw, bin(tt, j), LOGN + 1), j == 0 && !up,
+                        fs_untangle_self<(RE > 0 ? 1 : -1), R>(x + b * R, twiddle_big<S>(tw, bin(tt, j), LOGN + 1), j == 0 && !up,
                                                 [&](int r) {
                                                     const int k = j + r * NB;
                                                     return z[up ? L - 1 - k : (L - k) & (L - 1)];
@@ -672,15 +678,17 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             }
             each([&](int b, int tt, int j) {
                 if (!own(tt)) {
-                    fs_untangle<RE, R>(x + b * R, twiddle_big<RE>(tw, bin(tt, j), LOGN + 1), up);
+                    fs_untangle<(RE > 0 ? 1 : -1), R>(x + b * R, twiddle_big<S>(tw, bin(tt, j), LOGN + 1), up);
                     if (back)
 #pragma unroll
                         for (int r = R / 2; r < R; ++r) x[b * R + r] = fs_cross(x[b * R + r], up);
                 }
             });
         };
+        const bool second = RE != -2 && tr >= uint32_t(d.split);
+        const int64_t at = int64_t(second ? tr - uint32_t(d.split) : tr) * N;
         if (!t.b) {
-            const __amdgpu_buffer_rsrc_t rin = fs_rsrc(in + int64_t(tr) * N, uint32_t(N * CS));
+            const __amdgpu_buffer_rsrc_t rin = fs_rsrc((second ? in2 : in) + at, uint32_t(N * CS));
             // x[(j + r NB0) LB + idx TA + t]
             EA::template each_butterfly<0>(ltid, [&](int b, int tt, int j) {
                 constexpr int R = EA::R0, NB = LA / R;
@@ -702,6 +710,30 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                 f.load(tw, n2, jl, LOGN);
             };
             __builtin_amdgcn_s_setprio(1);
+            if constexpr (RE == -2) {
+                const __amdgpu_buffer_rsrc_t ry = fs_rsrc(in2 + at, uint32_t(N * CS));
+                constexpr T scale = (T)1 / (T)N;
+                EA::template each_butterfly<0>(ltid, [&](int b, int tt, int j) {
+                    constexpr int R = EA::R0, NB = LA / R, U = R < 8 ? R : 8;
+                    const uint32_t voff = (uint32_t(j * LB) + column(tt)) * uint32_t(CS);
+                    const bool dc = voff == 0;  // [F_0, F_N] in one slot
+#pragma unroll
+                    for (int r0 = 0; r0 < R; r0 += U) {
+                        cpx<T> y[U];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) y[u] = fs_load<T, FS_AUX_NT>(ry, voff, uint32_t((r0 + u) * NB * LB) * CS);
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            cpx<T>& x = v[b * R + r0 + u];
+                            const cpx<T> q = spec_apply(OP_CORREL, x, y[u], scale);
+                            if (r0 + u == 0)
+                                x = cpx<T>{dc ? spec_apply_real(OP_CORREL, x.x, y[u].x, scale) : q.x,
+                                           dc ? spec_apply_real(OP_CORREL, x.y, y[u].y, scale) : q.y};
+                            else x = q;
+                        }
+                    }
+                });
+            }
             if constexpr (RE < 0) {
                 untangle(
                     std::integral_constant<int, EA::R0>{}, std::integral_constant<int, LA>{}, v, ltid,
@@ -792,7 +824,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                     look(k);
                     __builtin_amdgcn_s_setprio(3);
                 });
-            const __amdgpu_buffer_rsrc_t ro = fs_rsrc(out + int64_t(tr) * N, uint32_t(N * CS));
+            const __amdgpu_buffer_rsrc_t ro = fs_rsrc((second ? out2 : out) + at, uint32_t(N * CS));
             if constexpr (RE > 0)
                 untangle(
                     std::integral_constant<int, EB::RL>{}, std::integral_constant<int, LB>{}, v, ltid,

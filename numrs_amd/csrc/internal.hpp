@@ -98,6 +98,7 @@ struct Launch {
     FsDesc fs{};          // LK_FUSED
     int src = B_IN;
     int dst = B_OUT;
+    int src2 = B_IN, dst2 = B_OUT;  // LK_FUSED: of the transforms from fs.split on
     int prec = 0;         // 0 = plain kernel, else split-precision MFMA kernel (MfmaPrec)
     // DMA-staged variant of an FP32 MODE_TT pass (k_c2c_dma), used when the
     // input pointer is 16-byte aligned; nullptr when the pass does not qualify.
@@ -211,14 +212,17 @@ struct FusedRef {
     const void* fn;
     int tiles_log;  // log2 tiles of one pass per transform
 };
-// real: the forward / inverse transform of 2^(logn + 1) reals.
-FusedRef fused_lookup_f32(int sign, int logn, bool real);
-FusedRef fused_lookup_f64(int sign, int logn, bool real);
+// FUSED_REAL: the forward / inverse transform of 2^(logn + 1) reals; FUSED_CORREL:
+// the same forward, the inverse of the correlation of two spectra.
+enum FusedForm { FUSED_C2C = 0, FUSED_REAL = 1, FUSED_CORREL = 2 };
+FusedRef fused_lookup_f32(int sign, int logn, int form);
+FusedRef fused_lookup_f64(int sign, int logn, int form);
 // The fused launch of `batch` transforms of 2^logn points from src to dst
 // with a ring of at most ring_bytes; false if the size has no such kernel or
-// runs faster as separate passes.  *ring_elems: complex values of its ring.
+// runs faster as separate passes (fewer tiles than `least`, or fused_min_tiles).
+// *ring_elems: complex values of its ring.
 bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size_t ring_bytes, Launch* l,
-                  size_t* ring_elems, bool real = false);
+                  size_t* ring_elems, int form = FUSED_C2C, int64_t least = 0);
 // Fewest tiles of a pass for the fused launch (its lead-in and its tail run
 // one pass only).  MI355X, buffers changing from call to call, fused against
 // separate passes: FP32 2^20 640 tiles 68.7 / 74.9 us, 512 tiles 58.7 / 60.1,
@@ -226,8 +230,8 @@ bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size
 // 63.7 / 68.3; FP64 2^18 768 tiles 74.9 / 75.9, 640 tiles 67.2 / 64.1.  Real, both
 // directions: FP32 2^19 640 tiles 167 / 170 us; 2^20 640 tiles 201 / 196, 1184 317 /
 // 392; 2^21 640 tiles 227 / 204, 1184 361 / 392.
-inline int64_t fused_min_tiles(bool f32, int logn, bool real) {
-    return (f32 ? real && logn >= 20 : logn >= 18) ? 1024 : 640;
+inline int64_t fused_min_tiles(bool f32, int logn, int form) {
+    return (f32 ? form != FUSED_C2C && logn >= 20 : logn >= 18) ? 1024 : 640;
 }
 constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;
 bool plan_is_fused(const Plan& p);
