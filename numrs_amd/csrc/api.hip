@@ -933,13 +933,14 @@ int host_c2c(int dtype, void* data, const std::vector<size_t>& nn, size_t batch,
     for (size_t v : nn) elems *= v;
     const size_t bytes = elems * csize(dtype);
     hipStream_t s = hipStreamPerThread;
-    DevBuf buf, tmp;
-    if ((rc = dev_alloc(buf, bytes, s))) return rc;
-    if ((rc = dev_alloc(tmp, p->tmp_elems * csize(dtype), s))) return rc;
-    HIPCHK(hipMemcpyAsync(buf.p, data, bytes, hipMemcpyHostToDevice, s));
-    if ((rc = exec_plan(*p, buf.p, buf.p, tmp.p, nullptr, isign, s))) return rc;
-    HIPCHK(hipMemcpyAsync(data, buf.p, bytes, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    const size_t tmp_bytes = p->tmp_elems * csize(dtype);
+    HostCall call(s);
+    call.open(bytes + tmp_bytes, 2);
+    void *buf, *tmp;
+    if ((rc = call.alloc(&buf, bytes)) || (rc = call.alloc(&tmp, tmp_bytes))) return rc;
+    if ((rc = call.upload(buf, data, bytes)) || (rc = call.started())) return rc;
+    if ((rc = exec_plan(*p, buf, buf, tmp, nullptr, isign, s))) return rc;
+    if ((rc = call.download(data, buf, bytes)) || (rc = call.finish())) return rc;
     return NRFFT_OK;
 }
 

@@ -168,6 +168,166 @@ void par_copy2d(char* dst, size_t dpitch, const char* src, size_t spitch, size_t
     });
 }
 
+// ---------------------------------------------------------------------------
+// Lanes of the host-pointer calls that are too small for the pipeline.
+//
+// What bounds them: the calls to the runtime.  Four hipMallocAsync and
+// hipFreeAsync take 65 us (2 KiB to 512 KiB), each transfer of pageable memory
+// about 12; so a lane's memory stays allocated, and small buffers move through
+// pinned memory by a copy kernel on the call's own stream (128 KiB in and out
+// around a kernel: 54 us against 64 by hipMemcpyAsync; 2 MiB: 227 and 225).  convlv
+// of 2^14 FP64 with 257 taps 122 -> 63 us (31 of them the kernel).
+// ---------------------------------------------------------------------------
+struct HostLane {
+    char* d = nullptr;
+    size_t cap = 0;
+    char* pin = nullptr;
+    bool busy = false;
+};
+
+namespace {
+
+constexpr size_t LANE_ALIGN = 256;
+constexpr size_t LANE_PIN = size_t(2) << 20, LANE_STAGED = size_t(1) << 20;  // staging, largest staged buffer
+size_t lane_round(size_t b) { return (b + LANE_ALIGN - 1) / LANE_ALIGN * LANE_ALIGN; }
+
+std::mutex g_lane_mu;
+HostLane g_lanes[64][HOST_LANES];
+
+// A lane of the current device with room for `bytes`, or nullptr.
+HostLane* lane_take(size_t bytes) {
+    int dev = 0;
+    if (bytes > HOST_LANE_MAX || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+    std::lock_guard<std::mutex> lk(g_lane_mu);
+    HostLane* best = nullptr;
+    for (HostLane& l : g_lanes[dev])
+        if (!l.busy && (!best || (best->cap < bytes && l.cap > best->cap))) best = &l;
+    if (!best) return nullptr;
+    if (best->cap < bytes) {
+        size_t cap = size_t(1) << 20;
+        while (cap < bytes) cap *= 2;
+        if (best->d) (void)hipFree(best->d);
+        best->d = nullptr;
+        best->cap = 0;
+        if (hipMalloc(reinterpret_cast<void**>(&best->d), cap) != hipSuccess) {
+            best->d = nullptr;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        best->cap = cap;
+    }
+    if (!best->pin && hipHostMalloc(reinterpret_cast<void**>(&best->pin), LANE_PIN, hipHostMallocDefault) != hipSuccess) {
+        best->pin = nullptr;  // transfers without staging
+        (void)hipGetLastError();
+    }
+    best->busy = true;
+    return best;
+}
+
+struct CopySegs {
+    const uint4* src[4];
+    uint4* dst[4];
+    uint32_t n[4];
+};
+// Up to four copies of n 16-byte words.
+__global__ __launch_bounds__(256) void k_host_copy(CopySegs c) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < c.n[k]; i += gridDim.x * 256) c.dst[k][i] = c.src[k][i];
+}
+
+}  // namespace
+
+void HostCall::open(size_t bytes, int buffers) { lane = lane_take(bytes + size_t(buffers) * LANE_ALIGN); }
+
+int HostCall::alloc(void** p, size_t bytes) {
+    *p = nullptr;
+    if (!bytes) return NRFFT_OK;
+    if (lane && used + lane_round(bytes) <= lane->cap) {
+        *p = lane->d + used;
+        used += lane_round(bytes);
+        return NRFFT_OK;
+    }
+    DevBuf b;
+    if (int rc = dev_alloc(b, bytes, s)) return rc;
+    *p = b.p;
+    own.push_back(b.p);
+    b.p = nullptr;
+    idle = false;
+    return NRFFT_OK;
+}
+
+// A place in the pinned staging for device buffer d, nullptr if it goes without
+// (only the lane's own buffers are padded to whole words of copy()).
+char* HostCall::stage(const void* d, size_t bytes) {
+    if (!lane || !lane->pin || d < lane->d || d >= lane->d + lane->cap || bytes > LANE_STAGED || staged + lane_round(bytes) > LANE_PIN || segs.size() == 4)
+        return nullptr;
+    char* p = lane->pin + staged;
+    staged += lane_round(bytes);
+    return p;
+}
+
+int HostCall::upload(void* dst, const void* src, size_t bytes) {
+    if (char* p = stage(dst, bytes)) {
+        std::memcpy(p, src, bytes);
+        segs.push_back(Seg{p, dst, bytes, nullptr});
+        return NRFFT_OK;
+    }
+    idle = false;
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+    return NRFFT_OK;
+}
+
+int HostCall::copy() {
+    if (segs.empty()) return NRFFT_OK;
+    CopySegs c{};
+    uint32_t most = 1;
+    for (size_t k = 0; k < segs.size(); ++k) {  // (whole 16-byte words: both sides are padded to LANE_ALIGN)
+        c.src[k] = static_cast<const uint4*>(segs[k].src);
+        c.dst[k] = static_cast<uint4*>(segs[k].dst);
+        c.n[k] = uint32_t((segs[k].bytes + 15) / 16);
+        most = std::max(most, c.n[k]);
+    }
+    idle = false;
+    hipLaunchKernelGGL(k_host_copy, dim3(std::min<uint32_t>(512, (most + 255) / 256)), dim3(256), 0, s, c);
+    HIPCHK(hipGetLastError());
+    return NRFFT_OK;
+}
+
+int HostCall::started() {
+    int rc = copy();
+    segs.clear();
+    idle = false;
+    return rc;
+}
+
+int HostCall::download(void* dst, const void* src, size_t bytes) {
+    if (char* p = stage(src, bytes)) {
+        segs.push_back(Seg{src, p, bytes, dst});
+        return NRFFT_OK;
+    }
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    return NRFFT_OK;
+}
+
+int HostCall::finish() {
+    if (int rc = copy()) return rc;
+    HIPCHK(hipStreamSynchronize(s));
+    idle = true;
+    for (const Seg& g : segs) std::memcpy(g.user, g.dst, g.bytes);
+    segs.clear();
+    return NRFFT_OK;
+}
+
+HostCall::~HostCall() {
+    if (lane && !idle) (void)hipStreamSynchronize(s);
+    for (void* p : own) (void)hipFreeAsync(p, s);
+    if (lane) {
+        std::lock_guard<std::mutex> lk(g_lane_mu);
+        lane->busy = false;
+    }
+}
+
 // Chunk i goes through slot i % ns: gathered on the host threads into the
 // pinned input slot, uploaded (stream 0), transformed (stream 1), downloaded
 // into the pinned output slot (stream 2) and scattered.  With two slots the

@@ -258,6 +258,40 @@ struct DevBuf {
     }
 };
 int dev_alloc(DevBuf& b, size_t bytes, hipStream_t s);
+// Device memory and transfers of one host-pointer call on stream s: open() with
+// the bytes of all its buffers, alloc() them, upload(), run, download(),
+// finish().  Calls of up to HOST_LANE_MAX bytes borrow a lane (a device block and
+// pinned staging, at most HOST_LANES a device, kept by the process); others, and
+// calls that find no lane free, allocate on the stream.
+constexpr size_t HOST_LANE_MAX = size_t(32) << 20;
+constexpr int HOST_LANES = 4;
+struct HostLane;
+struct HostCall {
+    explicit HostCall(hipStream_t st) : s(st) {}
+    ~HostCall();
+    void open(size_t bytes, int buffers);
+    int alloc(void** p, size_t bytes);
+    int upload(void* dst, const void* src, size_t bytes);
+    int started();  // before the transform: the staged uploads begin
+    int download(void* dst, const void* src, size_t bytes);
+    int finish();
+
+private:
+    struct Seg {
+        const void* src;
+        void* dst;
+        size_t bytes;
+        void* user;
+    };
+    int copy();
+    char* stage(const void* d, size_t bytes);
+    hipStream_t s;
+    HostLane* lane = nullptr;
+    size_t used = 0, staged = 0;
+    bool idle = true;  // nothing of this call is on the stream
+    std::vector<Seg> segs;
+    std::vector<void*> own;
+};
 // A batch of chunks streamed host -> HBM -> host through pinned staging:
 // gather(i, pinned) fills the input slot and returns its bytes; compute(i,
 // dev, ws, stream, &out, &out_bytes) transforms the uploaded chunk in the

@@ -538,17 +538,18 @@ int host_real(int kind, int dtype, const void* in, const void* aux, size_t aux_b
     if (rc) return rc;
     const size_t es = dtype == NRFFT_F32 ? 4 : 8;
     const size_t bytes = n * batch * es;
+    const size_t tmp = p->tmp_elems * csize(dtype);
     hipStream_t s = hipStreamPerThread;
-    DevBuf dbuf, dout, daux, dtmp;
-    if ((rc = dev_alloc(dbuf, bytes, s))) return rc;
-    if ((rc = dev_alloc(dout, bytes, s))) return rc;
-    if (aux_bytes && (rc = dev_alloc(daux, aux_bytes, s))) return rc;
-    if ((rc = dev_alloc(dtmp, p->tmp_elems * csize(dtype), s))) return rc;
-    HIPCHK(hipMemcpyAsync(dbuf.p, in, bytes, hipMemcpyHostToDevice, s));
-    if (aux_bytes) HIPCHK(hipMemcpyAsync(daux.p, aux, aux_bytes, hipMemcpyHostToDevice, s));
-    if ((rc = exec_plan(*p, dbuf.p, dout.p, dtmp.p, daux.p, isign, s))) return rc;
-    HIPCHK(hipMemcpyAsync(out, dout.p, bytes, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HostCall call(s);
+    call.open(2 * bytes + aux_bytes + tmp, 4);
+    void *dbuf, *dout, *daux, *dtmp;
+    if ((rc = call.alloc(&dbuf, bytes)) || (rc = call.alloc(&dout, bytes)) || (rc = call.alloc(&daux, aux_bytes)) ||
+        (rc = call.alloc(&dtmp, tmp)))
+        return rc;
+    if ((rc = call.upload(dbuf, in, bytes)) || (aux_bytes && (rc = call.upload(daux, aux, aux_bytes)))) return rc;
+    if ((rc = call.started())) return rc;
+    if ((rc = exec_plan(*p, dbuf, dout, dtmp, daux, isign, s))) return rc;
+    if ((rc = call.download(out, dout, bytes)) || (rc = call.finish())) return rc;
     return NRFFT_OK;
 }
 

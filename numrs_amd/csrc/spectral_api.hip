@@ -538,23 +538,24 @@ static int host_spectral(int kind, int dtype, std::vector<size_t> nn, HostBuf in
     int rc = cached_plan(kind, dtype, nn, 1, 0, &p);
     if (rc) return rc;
     hipStream_t s = hipStreamPerThread;
-    DevBuf dbin, daux, dout, daux2, dtmp;
     // `out` may be the same host buffer as `in` (in-place calls): then one
     // device buffer serves both.
     const bool same = out.dst != nullptr && out.dst == in.src;
-    if ((rc = dev_alloc(dbin, in.bytes, s))) return rc;
-    if (!same && out.bytes && (rc = dev_alloc(dout, out.bytes, s))) return rc;
-    if (aux.bytes && (rc = dev_alloc(daux, aux.bytes, s))) return rc;
-    if (aux2.bytes && (rc = dev_alloc(daux2, aux2.bytes, s))) return rc;
-    if ((rc = dev_alloc(dtmp, p->tmp_elems * csize(dtype), s))) return rc;
-    void* dout_p = same ? dbin.p : dout.p;
-    HIPCHK(hipMemcpyAsync(dbin.p, in.src, in.bytes, hipMemcpyHostToDevice, s));
-    if (aux.src) HIPCHK(hipMemcpyAsync(daux.p, aux.src, aux.bytes, hipMemcpyHostToDevice, s));
-    if (aux2.src) HIPCHK(hipMemcpyAsync(daux2.p, aux2.src, aux2.bytes, hipMemcpyHostToDevice, s));
-    if ((rc = exec_plan(*p, dbin.p, dout_p, dtmp.p, daux.p, isign, s, 0, -1, daux2.p))) return rc;
-    if (out.dst) HIPCHK(hipMemcpyAsync(out.dst, dout_p, out.bytes, hipMemcpyDeviceToHost, s));
-    if (aux2.dst) HIPCHK(hipMemcpyAsync(aux2.dst, daux2.p, aux2.bytes, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    const size_t tmp = p->tmp_elems * csize(dtype), ob = same ? 0 : out.bytes;
+    HostCall call(s);
+    call.open(in.bytes + ob + aux.bytes + aux2.bytes + tmp, 5);
+    void *dbin, *daux, *dout, *daux2, *dtmp;
+    if ((rc = call.alloc(&dbin, in.bytes)) || (rc = call.alloc(&dout, ob)) || (rc = call.alloc(&daux, aux.bytes)) ||
+        (rc = call.alloc(&daux2, aux2.bytes)) || (rc = call.alloc(&dtmp, tmp)))
+        return rc;
+    if (same) dout = dbin;
+    if ((rc = call.upload(dbin, in.src, in.bytes)) || (aux.src && (rc = call.upload(daux, aux.src, aux.bytes))) ||
+        (aux2.src && (rc = call.upload(daux2, aux2.src, aux2.bytes))) || (rc = call.started()))
+        return rc;
+    if ((rc = exec_plan(*p, dbin, dout, dtmp, daux, isign, s, 0, -1, daux2))) return rc;
+    if ((out.dst && (rc = call.download(out.dst, dout, out.bytes))) ||
+        (aux2.dst && (rc = call.download(aux2.dst, daux2, aux2.bytes))) || (rc = call.finish()))
+        return rc;
     return NRFFT_OK;
 }
 
