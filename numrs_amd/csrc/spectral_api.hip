@@ -322,7 +322,7 @@ int build_plan_spectral(Plan& p) {
             }
             if (fused) {
                 tag_launches(p, from, 1, 1);
-                const int64_t per = nn1 >= 2 ? nn1 * nn2 / 2 + 2 : nn2 / 2 + 1;  // row pairs of a volume
+                const int64_t per = nn1 >= 2 ? nn1 * nn2 / 2 : nn2 / 2;  // row pairs of a volume
                 Launch f = spec_launch(SP_R3_ROWS, B_TMP2, B_OUT, {batch * per, nn1, nn2, h});
                 f.args[7] = 1;
                 p.launches.push_back(f);
