@@ -185,11 +185,12 @@ __global__ __launch_bounds__(NT) void k_cosft1(const T* y, T* out, int64_t nsig,
     const int nvalid = (nsig - s0) < TI ? int(nsig - s0) : TI;
     const T* yb = y + s0 * S;
     if constexpr (LTM > 0) E::template stage_tw_to_lds<LTM>(ltw, tw.stage, tid);  // read after the first exchange
-    constexpr int PPT1 = (L / 2 + 1 + NT - 1) / NT;
+    // Bin pairs (p, L - p), p < L / 2; the thread of p = 0 takes the bins 0 and L / 2.
+    constexpr int NP = L / 2;
+    constexpr int PPT1 = (TI * NP + NT - 1) / NT;
     __shared__ cpx<T> uw[PPT1];
     PairTw<T, PPT1> ptw;
     if constexpr (TI == 1) ptw.init(uw, tw, tid, NT, LOG2N2);
-    constexpr int NP = L / 2 + 1;
     const T half = (T)0.5;
     if constexpr (cf1_persistent<T, L, TI, NT>()) {
         // Persistent over signals blockIdx.x + k gridDim.x, the next
@@ -204,17 +205,20 @@ __global__ __launch_bounds__(NT) void k_cosft1(const T* y, T* out, int64_t nsig,
         };
         auto finish = [&](int64_t sg) {
             T* os = out + sg * S;
-            int u = 0;
-            for (int p = tid; p < NP; p += NT, ++u) {
+#pragma unroll 1  // the next signal's values are in registers
+            for (int u = 0; u < PPT1; ++u) {
+                const int p = tid + u * NT;
+                if (NP % NT != 0 && p >= NP) break;
                 if (p == 0) {
                     const cpx<T> z0 = lds[E::lidx(0, 0)];
                     os[0] = half * (z0.x + z0.y);
                     os[L] = half * (z0.x - z0.y);
+                    os[NP] = half * lds[E::lidx(0, NP)].x;
                 } else {
                     cpx<T> fa, fb;
                     untangle_pair(lds[E::lidx(0, p)], lds[E::lidx(0, L - p)], ptw.at(uw, u), (T)-0.5, fa, fb);
                     os[p] = half * fa.x;
-                    if (L - p != p) os[L - p] = half * fb.x;
+                    os[L - p] = half * fb.x;
                 }
             }
         };
@@ -248,21 +252,24 @@ __global__ __launch_bounds__(NT) void k_cosft1(const T* y, T* out, int64_t nsig,
         const T* ys = yb + t * S;
         return cpx<T>{cf1_ext(ys, 2 * m, L), cf1_ext(ys, 2 * m + 1, L)};
     }, false, ltw);
-    int u = 0;
-    for (int q = tid; q < TI * NP; q += NT, ++u) {
-        const int t = q / NP, p = q % NP;
+#pragma unroll
+    for (int u = 0; u < PPT1; ++u) {
+        const int q = tid + u * NT;
+        if ((TI * NP) % NT != 0 && q >= TI * NP) break;
+        const int t = TI == 1 ? 0 : q / NP, p = TI == 1 ? q : q % NP;
         if (TI > 1 && t >= nvalid) continue;
         T* os = out + (s0 + t) * S;
         if (p == 0) {
             const cpx<T> z0 = lds[E::lidx(t, 0)];
             os[0] = half * (z0.x + z0.y);
             os[L] = half * (z0.x - z0.y);
+            os[NP] = half * lds[E::lidx(t, NP)].x;
         } else {
             cpx<T> fa, fb;
             const cpx<T> w = TI == 1 ? ptw.at(uw, u) : twiddle_big<1>(tw, (uint32_t)p, LOG2N2);
             untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], w, (T)-0.5, fa, fb);
             os[p] = half * fa.x;
-            if (L - p != p) os[L - p] = half * fb.x;
+            os[L - p] = half * fb.x;
         }
     }
 }
@@ -280,11 +287,15 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
     const int64_t s0 = int64_t(blockIdx.x) * TI;
     const int nvalid = (nsig - s0) < TI ? int(nsig - s0) : TI;
     const T* yb = y + s0 * N;
-    constexpr int NP = L / 2 + 1;
+    // Bin pairs (p, L - p), p < L / 2; the thread of p = 0 takes the packed slot
+    // and the self-paired bin L / 2, so that the loop has no round for one pair
+    // and, unrolled, its loads go out together (4096 x 2^14 FP32 inverse 146 us,
+    // forward 150; as a loop over L / 2 + 1 pairs 164 and 154).
+    constexpr int NP = L / 2;
     if constexpr (LTM > 0) E::template stage_tw_to_lds<LTM>(ltw, tw.stage, tid);  // read after the first exchange
     // One signal per group: untangle twiddles W_n^p and rotations W_4n^p,
     // W_4n^(L-p) = W_8 conj(W_4n^p) from per-thread and shared factors.
-    constexpr int PPT2 = (NP + NT - 1) / NT;
+    constexpr int PPT2 = (TI * NP + NT - 1) / NT;
     __shared__ cpx<T> uwn[PPT2], uw4[PPT2];
     PairTw<T, PPT2> pn, p4;
     cpx<T> w8{(T)0, (T)0};
@@ -293,6 +304,7 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
         p4.init(uw4, tw, tid, NT, LOGN + 2);
         w8 = twiddle_big<1>(tw, uint32_t(L), LOGN + 2);
     }
+    const cpx<T> w16{(T)0.92387953251128675612818318939679, (T)0.38268343236508977172845998403040};  // W_4n^(L/2)
     if constexpr (DIR > 0) {
         // The permuted gather stays element by element: through LDS in
         // 16-byte groups (as the inverse stores) it measured slower, 4096 x
@@ -302,39 +314,50 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
             const T* ys = yb + t * N;
             return cpx<T>{ys[cf2_pos(2 * m, L)], ys[cf2_pos(2 * m + 1, L)]};
         }, false, ltw);
-        int u = 0;
-        for (int q = tid; q < TI * NP; q += NT, ++u) {
-            const int t = q / NP, p = q % NP;
+#pragma unroll
+        for (int u = 0; u < PPT2; ++u) {
+            const int q = tid + u * NT;
+            if ((TI * NP) % NT != 0 && q >= TI * NP) break;
+            const int t = TI == 1 ? 0 : q / NP, p = TI == 1 ? q : q % NP;
             if (TI > 1 && t >= nvalid) continue;
             T* os = out + (s0 + t) * N;
             if (p == 0) {
                 const cpx<T> z0 = lds[E::lidx(t, 0)];
                 os[0] = z0.x + z0.y;
                 os[L] = (z0.x - z0.y) * cos_quarter_pi<T>();
+                cf2_fwd_out_w(w16, lds[E::lidx(t, NP)], NP, os, N);
             } else if constexpr (TI == 1) {
                 cpx<T> va, vb;
                 untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], pn.at(uwn, u), (T)-0.5, va, vb);
                 const cpx<T> r4 = p4.at(uw4, u);
                 cf2_fwd_out_w(r4, va, p, os, N);
-                if (L - p != p) cf2_fwd_out_w(cmul(w8, conj(r4)), vb, L - p, os, N);
+                cf2_fwd_out_w(cmul(w8, conj(r4)), vb, L - p, os, N);
             } else {
                 cpx<T> va, vb;
                 untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], twiddle_big<1>(tw, (uint32_t)p, LOGN),
                               (T)-0.5, va, vb);
                 cf2_fwd_out(tw, va, p, LOGN, os, N);
-                if (L - p != p) cf2_fwd_out(tw, vb, L - p, LOGN, os, N);
+                cf2_fwd_out(tw, vb, L - p, LOGN, os, N);
             }
         }
     } else {
         if constexpr (TI == 1) lds_barrier();  // uwn, uw4 published
-        int u = 0;
-        for (int q = tid; q < TI * NP; q += NT, ++u) {
-            const int t = q / NP, p = q % NP;
+        // (Several signals of 64 to 2048 bins a group: L / 2 + 1 pairs, whose odd count
+        // spreads the LDS writes; 2^8 FP32 197 us against 205.)
+        constexpr int NPI = TI > 1 && L >= 64 && L <= 2048 ? NP + 1 : NP;
+        constexpr int PPTI = (TI * NPI + NT - 1) / NT, UNR = TI == 1 ? PPTI : 1;
+#pragma unroll UNR
+        for (int u = 0; u < PPTI; ++u) {
+            const int q = tid + u * NT;
+            if ((TI * NPI) % NT != 0 && q >= TI * NPI) break;
+            const int t = TI == 1 ? 0 : q / NPI, p = TI == 1 ? q : q % NPI;
             const bool ok = TI == 1 || t < nvalid;
             const T* ys = yb + t * N;
             if (p == 0) {
                 const T sqrt2 = (T)1.41421356237309504880;
                 lds[E::lidx(t, 0)] = ok ? dc_inverse(cpx<T>{ys[0], sqrt2 * ys[L]}) : cpx<T>{(T)0, (T)0};
+                if (NPI == NP)
+                    lds[E::lidx(t, NP)] = ok ? cmul(conj(w16), cpx<T>{ys[NP], ys[N - NP]}) : cpx<T>{(T)0, (T)0};
             } else {
                 cpx<T> za{(T)0, (T)0}, zb{(T)0, (T)0};
                 if constexpr (TI == 1) {
