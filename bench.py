@@ -6,10 +6,10 @@ isign = +1, inputs resident in HBM, out of place.  One step = one plan
 execution over the whole batch.  GFLOP/s uses 5 N log2 N per transform.
 
 The same line carries
-  roofline:      the dominant kernel (slower four-step pass), algorithmic bytes
-                 per launch (one read + one write of its chunk, 16 B per
-                 point) / its average duration between HIP events recorded
-                 after every launch of the plan, in sequence, on its stream;
+  roofline:      the kernel of the step (k_fused4: both four-step passes in one
+                 launch), algorithmic bytes per launch (one read + one write
+                 of the batch, 16 B per point) / its average duration between
+                 HIP events recorded around every step on its stream;
   cpu_baseline:  the oracle's restatement of FFT_1::four1 (FP64, OpenMP over
                  transforms like FFTProcessor::fft_batch) timed on the host
                  cores on a bounded sample of the same workload;
@@ -79,18 +79,16 @@ def time_events(fn, reps: int) -> float:
 
 
 def measured_traffic_ratio():
-    """Bytes past L2 / algorithmic bytes of the FP32 four-step passes, from the
+    """Bytes past L2 / algorithmic bytes of the FP32 fused four-step, from the
     committed rocprofv3 summary of raw TCC request counts (last column)."""
     path = os.path.join(ROOT, "profiles", "c2c_fp32_batch64_n2p20_traffic.txt")
     try:
-        ratios = []
         for line in open(path):
-            parts = line.split()
-            if line.startswith(" nrfft::k_c2c_dma<1, 512>") or line.startswith(" nrfft::k_c2c<float, 1, 2048"):
-                ratios.append(float(parts[-1]))
-        return (max(ratios), os.path.relpath(path, ROOT)) if ratios else (None, None)
+            if line.startswith(" nrfft::k_fused4<float, 1, 1024, 1024, 0>"):
+                return float(line.split()[-1]), os.path.relpath(path, ROOT)
     except (OSError, ValueError):
-        return None, None
+        pass
+    return None, None
 
 
 def _rel_l2_gpu(a, ref) -> float:
@@ -127,6 +125,22 @@ def _time_plan(plan, x, y, steps: int, warmup: int, settle: float = 1.0) -> floa
     return (time.perf_counter() - t0) * 1e3 / steps
 
 
+def _time_steps_in_sequence(plan, x, y, steps: int) -> float:
+    """Average ms of an execution between consecutive HIP events in `steps`
+    back-to-back executions."""
+    import torch
+
+    s = torch.cuda.current_stream()
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(steps + 1)]
+    torch.cuda.synchronize()
+    ev[0].record(s)
+    for st in range(steps):
+        plan.execute(x, y, 1)
+        ev[st + 1].record(s)
+    torch.cuda.synchronize()
+    return sum(ev[st].elapsed_time(ev[st + 1]) for st in range(steps)) / steps
+
+
 def _time_launches_in_sequence(plan, x, y, steps: int) -> list:
     """Average ms of each launch of the plan, measured between consecutive
     HIP events in `steps` back-to-back executions."""
@@ -159,25 +173,19 @@ def headline(args) -> dict:
     fill_uniform(x, 3, 0, 2 * pts)
     plan = numrs_amd.C2CPlan("float32", [n], batch)
     nl = plan.num_launches
-    log(f"[bench] timing {args.steps} steps ({nl} launches per step)")
+    log(f"[bench] timing {args.steps} steps")
     ms = _time_plan(plan, x, y, args.steps, args.warmup)
     flops = 5.0 * n * logn * batch
     gflops = flops / (ms * 1e-3) / 1e9
     compulsory = 2.0 * pts * 8  # one read + one write, 8 B per complex
-    # Per-launch durations: the plan's launches issued one by one in their
-    # normal order for `steps` more steps, with a HIP event recorded after
-    # each on the stream the library launches on (torch's current stream), so
-    # every launch is timed inside the real sequence (the chunk written by
-    # pass A is what pass B reads).  Four-step plans alternate pass A / pass B
-    # over batch chunks; each launch reads and writes every point of its
-    # chunk once.
+    # The step is one launch: its duration between HIP events recorded around
+    # `steps` more back-to-back steps on the stream the library launches on
+    # (torch's current stream).  The plan's pass-by-pass form (pass A / pass B
+    # over batch chunks, what execute_launches issues) is timed beside it.
+    kernel_ms = _time_steps_in_sequence(plan, x, y, args.steps)
     per = _time_launches_in_sequence(plan, x, y, args.steps)
-    kinds = ["A", "B"] if nl % 2 == 0 and nl > 1 else ["pass"]
-    groups = {k: [per[i] for i in range(nl) if kinds[i % len(kinds)] == k] for k in kinds}
-    dom = max(groups, key=lambda k: sum(groups[k]))
-    launch_bytes = compulsory / (nl // len(kinds))
-    dom_ms = sum(groups[dom]) / len(groups[dom])
-    achieved = launch_bytes / (dom_ms * 1e-3) / 1e9
+    plan.execute(x, y, 1)
+    achieved = compulsory / (kernel_ms * 1e-3) / 1e9
     ratio, tsrc = measured_traffic_ratio()
     out = {
         "metric": METRIC,
@@ -193,24 +201,23 @@ def headline(args) -> dict:
         "dtype": "f32",
         "data": "synthetic: re/im i.i.d. uniform[-1,1) from SplitMix64 seed 3",
         "config": {"workload": "four1 C2C FP32, batch 64 x N=2^20, isign=+1, out of place, HBM-resident",
-                   "batch": batch, "n": n, "launches": nl, "parallelism": "single-gpu"},
+                   "batch": batch, "n": n, "launches": 1, "parallelism": "single-gpu"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": int(ratio * launch_bytes) if ratio else None,
+                     "traffic": int(ratio * compulsory) if ratio else None,
                      "traffic_source": tsrc,
-                     # FP32 pass A over 512-point columns runs as k_c2c_dma (16-byte aligned input)
-                     "kernel": f"four-step pass {dom} ({'k_c2c_dma' if dom == 'A' else 'k_c2c'}), "
-                               f"{len(groups[dom])} launches per step",
-                     "kernel_ms": round(dom_ms, 4), "algorithmic_bytes_per_launch": int(launch_bytes)},
+                     "kernel": "k_fused4<float, 1, 1024, 1024>, 1 launch per step",
+                     "kernel_ms": round(kernel_ms, 4), "algorithmic_bytes_per_launch": int(compulsory)},
         "hbm_effective": {"GBps": round(compulsory / (ms * 1e-3) / 1e9, 1),
                           "frac": round(compulsory / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                           "note": "compulsory bytes (one read + one write of the batch) / whole step"},
-        "traffic_rate": ({"GBps": round(ratio * launch_bytes * nl / (ms * 1e-3) / 1e9, 1),
-                          "frac": round(ratio * launch_bytes * nl / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+        "traffic_rate": ({"GBps": round(ratio * compulsory / (ms * 1e-3) / 1e9, 1),
+                          "frac": round(ratio * compulsory / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                           "note": "counter-measured bytes past L2 per step (rocprofv3 TCC read / write request "
-                                  "counts of every launch, from traffic_source) / whole step; each of the two "
-                                  "passes reads and writes every point"} if ratio else None),
-        "launch_ms": [round(p, 4) for p in per],
+                                  "counts, from traffic_source) / whole step; the intermediate's share stays in "
+                                  "the last-level cache"} if ratio else None),
+        "launch_ms": [round(kernel_ms, 4)],
+        "separate_passes": {"launches": nl, "ms": round(sum(per), 4), "launch_ms": [round(p, 4) for p in per]},
     }
     # FP64 reference of the same FP32 inputs from the FP64 path (parity-tested
     # against the oracle at 1e-12), for the relative L2 of every FP32 form.
@@ -228,7 +235,7 @@ def headline(args) -> dict:
     out["fp64"] = {"ms": round(ms64, 4), "GFLOPs": round(flops / (ms64 * 1e-3) / 1e9, 1),
                    "GBps_compulsory": round(comp64 / (ms64 * 1e-3) / 1e9, 1),
                    "frac_hbm": round(comp64 / (ms64 * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                   "launches": p64.num_launches}
+                   "launches": 1}
     del x64, y64b, p64
     split = {}
     for name in ("f16", "bf16"):
@@ -815,7 +822,7 @@ def _extra_uneven() -> dict:
         "max_rel_l2_vs_fp64": worst, "rel_l2_all_vs_fp64": math.sqrt(acc_e / acc_r),
         "tasks": [info["tasks_phase1"], info["tasks_phase2"]], "groups": info["groups"],
         "autotuned_split_log2_n1": {str(k): v[0] for k, v in tuned.items()},
-        "launch": "graph replay: counter-reset fill kernel + the persistent queue kernel, one dispatch per pass phase"}
+        "launch": "graph replay of the persistent queue kernel, one dispatch"}
     return res
 
 

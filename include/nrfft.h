@@ -226,7 +226,7 @@ typedef struct nrfft_uneven_s* nrfft_uneven;
 int nrfft_plan_uneven(nrfft_uneven* plan, int dtype, size_t nitems, const int* ndim, const size_t* dims,
                       const size_t* offs);
 int nrfft_execute_uneven(nrfft_uneven plan, const void* d_in, void* d_out, int isign, void* stream);
-/* Same work as plain launches (reset, phase 1, phase 2) instead of a graph replay. */
+/* Same work as a plain launch instead of a graph replay. */
 int nrfft_execute_uneven_nograph(nrfft_uneven plan, const void* d_in, void* d_out, int isign, void* stream);
 /* Waits for the stream and reports NRFFT_E_HIP if the last execution left tasks untaken. */
 int nrfft_uneven_check(nrfft_uneven plan, void* stream);
