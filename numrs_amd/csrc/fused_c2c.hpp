@@ -14,7 +14,7 @@
 // MI355X (random data; 2 GiB past the L2s, 7.2 TB/s), this kernel 324.  Two
 // launches per batch chunk (k_c2c_dma / k_c2c) took 445: each pays a ramp and a
 // drain, and their chunks have to be 64-128 MiB to fill the chip, so input,
-// intermediate and output share the MALL.  FP64 45 x 2^18 150 -> 126 us.
+// intermediate and output share the MALL.  FP64 45 x 2^18 150 -> 124 us.
 //
 // Groups take work from one ticket counter.  A ticket is a unit: A tile u,
 // then B tile u - lead, with lead = `lag` slabs; a slab is 64 tiles

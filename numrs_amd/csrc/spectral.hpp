@@ -345,11 +345,7 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
         // (Several signals of 64 to 2048 bins a group: L / 2 + 1 pairs, whose odd count
         // spreads the LDS writes; 2^8 FP32 197 us against 205.)
         constexpr int NPI = TI > 1 && L >= 64 && L <= 2048 ? NP + 1 : NP;
-        constexpr int PPTI = (TI * NPI + NT - 1) / NT, UNR = TI == 1 ? PPTI : 1;
-#pragma unroll UNR
-        for (int u = 0; u < PPTI; ++u) {
-            const int q = tid + u * NT;
-            if ((TI * NPI) % NT != 0 && q >= TI * NPI) break;
+        auto pair = [&](int u, int q) {
             const int t = TI == 1 ? 0 : q / NPI, p = TI == 1 ? q : q % NPI;
             const bool ok = TI == 1 || t < nvalid;
             const T* ys = yb + t * N;
@@ -372,6 +368,22 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
                 lds[E::lidx(t, p)] = za;
                 lds[E::lidx(t, L - p)] = zb;
             }
+        };
+        if constexpr (TI == 1) {
+            constexpr int PPTI = (NPI + NT - 1) / NT;
+#pragma unroll
+            for (int u = 0; u < PPTI; ++u)
+                if (NPI % NT == 0 || tid + u * NT < NPI) pair(u, tid + u * NT);
+        } else if constexpr (NPI == NP) {
+            constexpr int PPTI = (TI * NPI + NT - 1) / NT;
+#pragma unroll 1
+            for (int u = 0; u < PPTI; ++u) {
+                if ((TI * NPI) % NT != 0 && tid + u * NT >= TI * NPI) break;
+                pair(u, tid + u * NT);
+            }
+        } else {
+            int u = 0;
+            for (int q = tid; q < TI * NPI; q += NT, ++u) pair(u, q);
         }
         lds_barrier();
         if constexpr (TI == 1 && CF2_LDS) {
