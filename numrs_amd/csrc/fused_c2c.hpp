@@ -29,7 +29,8 @@
 // against 293 with plain stores).  A group that has waited for its stores
 // counts its tile in the slab's counter; a B tile starts once the counter has
 // reached the slab's tiles.  An A tile that reuses a slot starts once the B
-// tiles of the slab that was there have all loaded.  A tile depends only on
+// tiles of the slab that was there have all loaded: one thread counts a B tile
+// behind the first barrier of its exchange, which no wave passes without its values.  A tile depends only on
 // units with smaller tickets, and a group that holds a ticket runs, so the
 // smallest unfinished unit never waits: no deadlock, however few groups are
 // resident.  Every wait is bounded all the same (a group polls FS_SPIN times in
@@ -297,17 +298,21 @@ struct FsEng {
 #pragma unroll
         for (int b = 0; b < EPT / R; ++b) fs_dft<R, S>(v + b * R);
     }
-    // Stages 1 .. NST-1; stage 0's outputs are in v.  Hooks in the last exchange:
-    // `pre` before it, `mid` behind its first barrier, `late` before its last read.
-    template <int s = 1, class LTW, class PRE, class MID, class LATE>
-    static __device__ __forceinline__ void rest(cpx<T>* v, int tid, T* ex, LTW ltw, const cpx<T>* stage_tw, PRE&& pre,
-                                                MID&& mid, LATE&& late) {
+    // Stages 1 .. NST-1; stage 0's outputs are in v.  Hook behind the first
+    // exchange's first barrier: `read`; there every wave has written outputs of all
+    // its stage-0 butterflies, so each value the group loaded has arrived.  Hooks in
+    // the last exchange: `pre` before it, `mid` behind its first barrier, `late`
+    // before its last read.
+    template <int s = 1, class LTW, class READ, class PRE, class MID, class LATE>
+    static __device__ __forceinline__ void rest(cpx<T>* v, int tid, T* ex, LTW ltw, const cpx<T>* stage_tw, READ&& read,
+                                                PRE&& pre, MID&& mid, LATE&& late) {
         static_assert(NST == 2 || std::is_base_of_v<FsTablePlan<L>, P>, "stage 2 reads the per-stage table");
         if constexpr (s < NST) {
             if constexpr (s > 1) lds_barrier();  // the previous exchange has been read
             if constexpr (s == NST - 1) pre();
             put<s - 1, 0>(v, tid, ex);
             lds_barrier();
+            if constexpr (s == 1) read();
             if constexpr (s == NST - 1) mid();
             get<s, 0>(v, tid, ex);
             lds_barrier();
@@ -317,7 +322,7 @@ struct FsEng {
             get<s, 1>(v, tid, ex);
             twiddle<s>(v, tid, ltw, stage_tw);
             butterflies<s>(v);
-            rest<s + 1>(v, tid, ex, ltw, stage_tw, pre, mid, late);
+            rest<s + 1>(v, tid, ex, ltw, stage_tw, read, pre, mid, late);
         }
     }
 };
@@ -414,6 +419,10 @@ __device__ __forceinline__ uint32_t fs_peek(const uint32_t* p) {
 __device__ __forceinline__ void fs_count(uint32_t* p) {
     __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Where a ring slot's tile is counted as loaded: the next tile's stores to the slot
+// may follow.  (The comment marks the place in the assembly, where
+// tests/test_ring_release.py finds every load from the ring waited for.)
+__device__ __forceinline__ void fs_release_mark() { asm volatile("; ring slot released" ::: "memory"); }
 
 // ---------------------------------------------------------------------------
 // The untangle of a real transform (untangle_pair, real_fft.hpp) on mirror pairs
@@ -533,7 +542,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
     __shared__ __align__(16) T ex[SH::EX];
     __shared__ __align__(16) cpx<T> ltwa[SH::TWA];
     __shared__ __align__(16) cpx<T> ltwb_[SH::TWB];
-    __shared__ uint32_t sh[2], arrive[2];
+    __shared__ uint32_t sh[2], arrive;
     const cpx<T>* ltwb = SH::SAME_TW ? ltwa : ltwb_;
     const int tid = threadIdx.x;
 
@@ -586,7 +595,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             if (next < 2 * units) seen = fs_peek(waits_on(task_of(next)));
         }
     };
-    if (tid < 2) arrive[tid] = 0;  // (before the first barrier)
+    if (tid == 0) arrive = 0;  // (before the first barrier)
     take_ticket();
     EA::fill_tw(ltwa, tw.coarse, tid);
     if constexpr (!SH::SAME_TW) EB::fill_tw(ltwb_, tw.coarse, tid);
@@ -635,8 +644,8 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
         auto publish = [&]() {
             if (!pending) return;
             fs_drain<EPT>();
-            if ((tid & 63) == 0 && atomicAdd(&arrive[0], 1u) == FS_NT / 64 - 1) {
-                arrive[0] = 0;
+            if ((tid & 63) == 0 && atomicAdd(&arrive, 1u) == FS_NT / 64 - 1) {
+                arrive = 0;
                 fs_count(pending);
             }
         };
@@ -742,7 +751,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             }
             EA::template butterflies<0>(v);
             EA::rest(
-                v, ltid, ex, typename EA::Ltw{ltwa}, tw.stage, load_tw,
+                v, ltid, ex, typename EA::Ltw{ltwa}, tw.stage, []() {}, load_tw,
                 [&]() {
                     __builtin_amdgcn_s_setprio(2);
                     f.join();
@@ -813,13 +822,13 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
             if (last_of_unit(k)) take_ticket();
             __builtin_amdgcn_s_setprio(1);
             EB::template butterflies<0>(v);
-            // Likewise the last wave that has its values counts the tile as loaded.
-            if ((tid & 63) == 0 && atomicAdd(&arrive[1], 1u) == FS_NT / 64 - 1) {
-                arrive[1] = 0;
-                fs_count(st->loaded[t.slot]);
-            }
             EB::rest(
-                v, ltid, ex, typename EB::Ltw{ltwb}, tw.stage, []() {}, []() { __builtin_amdgcn_s_setprio(2); },
+                v, ltid, ex, typename EB::Ltw{ltwb}, tw.stage,
+                [&]() {
+                    fs_release_mark();
+                    if (tid == 0) fs_count(st->loaded[t.slot]);
+                },
+                []() {}, []() { __builtin_amdgcn_s_setprio(2); },
                 [&]() {
                     look(k);
                     __builtin_amdgcn_s_setprio(3);

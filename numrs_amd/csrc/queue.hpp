@@ -102,8 +102,8 @@ constexpr int q_ex_elems() {
     }
 }
 
-// One tile.  publish: after its loads are issued; loaded: they have arrived;
-// mid / late: FsEng's hooks.
+// One tile.  publish: after its loads are issued; loaded: every wave's have
+// arrived (FsEng's hook `read`); mid / late: FsEng's hooks.
 template <typename T, int S, int C, class PUB, class LOADED, class MID, class LATE>
 __device__ __forceinline__ void q_tile(const QTask& q, const cpx<T>* in, cpx<T>* out, cpx<T>* ring,
                                        const uint32_t* __restrict__ offs, T* ex,
@@ -149,7 +149,6 @@ __device__ __forceinline__ void q_tile(const QTask& q, const cpx<T>* in, cpx<T>*
         publish();
         __builtin_amdgcn_s_setprio(1);
         E::template butterflies<0>(v);
-        if constexpr (MODE == Q_RING) loaded();
         FsTw<T, S, E::RL, EPT / E::RL, E::NBL> f;
         uint32_t at1[EPT / E::RL];  // where the outputs go
         auto load_tw = [&]() {
@@ -165,7 +164,11 @@ __device__ __forceinline__ void q_tile(const QTask& q, const cpx<T>* in, cpx<T>*
             }
         };
         E::rest(
-            v, tid, ex, q_ltw<T, E::P::R[1], E::ns(1)>(ltw), tw.stage, load_tw,
+            v, tid, ex, q_ltw<T, E::P::R[1], E::ns(1)>(ltw), tw.stage,
+            [&]() {
+                if constexpr (MODE == Q_RING) loaded();
+            },
+            load_tw,
             [&]() {
                 __builtin_amdgcn_s_setprio(2);
                 if constexpr (MODE == Q_COL) f.join();
@@ -204,7 +207,7 @@ k_queue(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, const QTask* __restrict__ t
         const uint32_t* __restrict__ offs, uint32_t* ctr, const uint32_t* __restrict__ init, int lines, Twiddles<T> tw) {
     __shared__ __align__(16) T ex[q_ex_elems<T>()];
     __shared__ __align__(16) cpx<T> ltw[q_tw_elems<T>()];
-    __shared__ uint32_t sh[2], arrive[2];
+    __shared__ uint32_t sh[2], arrive;
     static_assert(sizeof(ex) + sizeof(ltw) + 64 <= 81920, "two groups share a CU");
     const int tid = threadIdx.x;
     const bool wave0 = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
@@ -228,7 +231,7 @@ k_queue(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, const QTask* __restrict__ t
             next_n = tasks[next].nwait;
         }
     };
-    if (tid < 2) arrive[tid] = 0;
+    if (tid == 0) arrive = 0;
     take_ticket();
     q_fill_tw(ltw, tw.coarse, tid);
     if (wave0) aim(2u * __builtin_amdgcn_readfirstlane(taken));
@@ -268,18 +271,16 @@ k_queue(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, const QTask* __restrict__ t
         auto publish = [&]() {
             if (pending) {
                 fs_drain<fs_ept<T>()>();
-                if ((tid & 63) == 0 && atomicAdd(&arrive[0], 1u) == FS_NT / 64 - 1) {
-                    arrive[0] = 0;
+                if ((tid & 63) == 0 && atomicAdd(&arrive, 1u) == FS_NT / 64 - 1) {
+                    arrive = 0;
                     q_count(pending);
                 }
             }
             if (last) take_ticket();
         };
         auto loaded = [&]() {
-            if (q.count && (tid & 63) == 0 && atomicAdd(&arrive[1], 1u) == FS_NT / 64 - 1) {
-                arrive[1] = 0;
-                q_count(line(q.count));
-            }
+            fs_release_mark();
+            if (tid == 0) q_count(line(q.count));
         };
         auto mid = [&]() {
             if (wave0) aim(last ? 2u * __builtin_amdgcn_readfirstlane(taken) : uint32_t(k) + 1);
