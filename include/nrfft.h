@@ -154,6 +154,8 @@ int nrfft_execute_correl(nrfft_plan plan, const void* d_data1, const void* d_dat
  * stream do not.  In place allowed (d_out == d_in). */
 int nrfft_execute_four1_batch_noalloc(int dtype, const void* d_in, void* d_out, size_t nn, size_t batch, int isign,
                                       void* stream);
+/* nrfft_plan_check for the calls above, on the current device. */
+int nrfft_four1_batch_noalloc_check(void* stream);
 
 /* Profiling aid (no counterpart in the reference): enqueue only launches
  * [first, first + count) of a C2C plan, e.g. one pass of a four-step plan. */
@@ -228,8 +230,11 @@ int nrfft_plan_uneven(nrfft_uneven* plan, int dtype, size_t nitems, const int* n
 int nrfft_execute_uneven(nrfft_uneven plan, const void* d_in, void* d_out, int isign, void* stream);
 /* Same work as a plain launch instead of a graph replay. */
 int nrfft_execute_uneven_nograph(nrfft_uneven plan, const void* d_in, void* d_out, int isign, void* stream);
-/* Waits for the stream and reports NRFFT_E_HIP if the last execution left tasks untaken. */
+/* Waits for the stream and reports NRFFT_E_HIP if the last execution left tasks untaken
+ * or a wait inside one gave up since the last check (nrfft_plan_check). */
 int nrfft_uneven_check(nrfft_uneven plan, void* stream);
+/* As nrfft_plan_launch_info; ring_reused: 1 if parts of the ring serve several items. */
+int nrfft_uneven_launch_info(nrfft_uneven plan, int* launches, int* ring_reused, void** expired);
 int nrfft_uneven_info(nrfft_uneven plan, size_t* tasks_phase1, size_t* tasks_phase2, size_t* workspace_bytes,
                       unsigned* groups);
 int nrfft_uneven_destroy(nrfft_uneven plan);
@@ -286,6 +291,18 @@ size_t nrfft_plan_workspace_bytes(nrfft_plan plan);
  * nrfft_execute_c2c may run both four-step passes of a 1-D plan, all chunks, as
  * one launch instead (same result up to rounding). */
 int nrfft_plan_num_launches(nrfft_plan plan);
+/* A launch that runs several passes holds waits between its tiles, each given up
+ * after about a second (something kept part of the launch off the GPU, or the plan
+ * ran on two streams at once); the results of that execution are then not valid.
+ * Waits for the stream and reports NRFFT_E_HIP if that happened since the plan was
+ * made or last checked; NRFFT_OK for plans without such a launch. */
+int nrfft_plan_check(nrfft_plan plan, void* stream);
+/* What one execution in direction isign enqueues: *launches kernels and copies;
+ * *ring_slabs slabs of work through *ring_slots places of the ring of a launch that
+ * runs several passes (0, 0: no such launch); *expired: the device address of the
+ * 32-bit word that is not 0 once a wait has given up (NULL: none).  Any may be NULL. */
+int nrfft_plan_launch_info(nrfft_plan plan, int isign, int* launches, int* ring_slots, int* ring_slabs,
+                           void** expired);
 
 #ifdef __cplusplus
 }

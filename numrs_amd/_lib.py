@@ -108,6 +108,11 @@ _SIGS = {
     "nrfft_plan_destroy": (_i, [_vp]),
     "nrfft_plan_workspace_bytes": (_sz, [_vp]),
     "nrfft_plan_num_launches": (_i, [_vp]),
+    "nrfft_plan_check": (_i, [_vp, _vp]),
+    "nrfft_plan_launch_info": (_i, [_vp, _i, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_i),
+                                    ctypes.POINTER(_vp)]),
+    "nrfft_four1_batch_noalloc_check": (_i, [_vp]),
+    "nrfft_uneven_launch_info": (_i, [_vp, ctypes.POINTER(_i), ctypes.POINTER(_i), ctypes.POINTER(_vp)]),
 }
 
 _lib = None

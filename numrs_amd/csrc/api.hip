@@ -126,6 +126,17 @@ void fs_state_give(int device, FsState* st) {
     if (st && it != g_ctx.end()) it->second->fs_free.push_back(st);  // capacity reserved: does not throw
 }
 
+int expired_check(uint32_t* d_word, hipStream_t s) {
+    uint32_t word = 0;
+    HIPCHK(hipMemcpyAsync(&word, d_word, sizeof word, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (!word) return NRFFT_OK;
+    word = 0;
+    HIPCHK(hipMemcpyAsync(d_word, &word, sizeof word, hipMemcpyHostToDevice, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return fail(NRFFT_E_HIP, "a wait inside a persistent launch gave up: results since the last check are not valid");
+}
+
 // The current device's context if nrfft_init (or any earlier call) built
 // it; never allocates.
 int find_ctx(DeviceCtx** out) {
@@ -1180,5 +1191,36 @@ int nrfft_plan_destroy(nrfft_plan plan) {
 size_t nrfft_plan_workspace_bytes(nrfft_plan plan) { return plan ? plan->tmp_bytes : 0; }
 
 int nrfft_plan_num_launches(nrfft_plan plan) { return plan ? (int)plan->plan.launches.size() : 0; }
+
+int nrfft_plan_check(nrfft_plan plan, void* stream) {
+    g_err.clear();
+    if (!plan) return fail(NRFFT_E_INVALID, "null plan");
+    if (!plan->plan.fs_state) return NRFFT_OK;
+    return expired_check(&plan->plan.fs_state->expired, (hipStream_t)stream);
+}
+
+int nrfft_plan_launch_info(nrfft_plan plan, int isign, int* launches, int* ring_slots, int* ring_slabs,
+                           void** expired) {
+    g_err.clear();
+    if (!plan) return fail(NRFFT_E_INVALID, "null plan");
+    if (isign != 1 && isign != -1) return fail(NRFFT_E_ISIGN, "isign must be 1 or -1");
+    const Plan& p = plan->plan;
+    int count = 0, slots = 0, slabs = 0;
+    for (const Launch& l : p.whole.empty() ? p.launches : p.whole) {
+        if (l.args[7] != 0 && (l.args[7] > 0) != (isign > 0)) continue;  // the other direction's
+        ++count;
+        if (l.kind != LK_FUSED) continue;
+        const int s = (l.fs.batch + (1 << l.fs.slab_log) - 1) >> l.fs.slab_log;
+        if (s > slabs) {
+            slabs = s;
+            slots = l.fs.slots;
+        }
+    }
+    if (launches) *launches = count;
+    if (ring_slots) *ring_slots = slots;
+    if (ring_slabs) *ring_slabs = slabs;
+    if (expired) *expired = p.fs_state ? &p.fs_state->expired : nullptr;
+    return NRFFT_OK;
+}
 
 }  // extern "C"

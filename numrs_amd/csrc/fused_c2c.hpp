@@ -34,8 +34,9 @@
 // units with smaller tickets, and a group that holds a ticket runs, so the
 // smallest unfinished unit never waits: no deadlock, however few groups are
 // resident.  Every wait is bounded all the same (a group polls FS_SPIN times in
-// vain at most once), so misuse (one plan on two streams at once) gives wrong
-// results, not a hang.
+// vain at most once, about a second), so misuse (one plan on two streams at once)
+// gives wrong results, not a hang.  A group that gives up sets `expired`, which
+// stays set until a check reads it (nrfft_plan_check).
 //
 // The last group to leave clears the counters, so a launch leaves the state
 // as it found it and needs no reset launch or memset before it.  (The count of
@@ -52,10 +53,12 @@ constexpr int FS_MAX_SLOTS = 32;
 constexpr int FS_SPIN = 1 << 20;
 
 // Counters of a fused plan, each on a cache line of its own (operations on
-// one line queue up behind each other).  All zero between launches.
+// one line queue up behind each other).  All but `expired` are zero between
+// launches.
 struct FsState {
-    uint32_t ticket, pad0[31];
-    uint32_t done, pad1[31];
+    uint32_t expired, pad0[31];  // a wait has given up
+    uint32_t ticket, pad1[31];
+    uint32_t done, pad2[31];
     uint32_t stored[FS_MAX_SLOTS][32];  // [slot][0]: A tiles of the slot's slabs that are stored
     uint32_t loaded[FS_MAX_SLOTS][32];  // [slot][0]: B tiles of the slot's slabs that are loaded
 };
@@ -419,6 +422,9 @@ __device__ __forceinline__ uint32_t fs_peek(const uint32_t* p) {
 __device__ __forceinline__ void fs_count(uint32_t* p) {
     __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void fs_flag(uint32_t* p) {
+    __hip_atomic_store(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // Where a ring slot's tile is counted as loaded: the next tile's stores to the slot
 // may follow.  (The comment marks the place in the assembly, where
 // tests/test_ring_release.py finds every load from the ring waited for.)
@@ -629,7 +635,10 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
                     if (__builtin_amdgcn_readfirstlane(fs_peek(p)) >= need) break;
                     __builtin_amdgcn_s_sleep(8);
                 }
-                if (i == patience) patience = 0;
+                if (i == patience) {
+                    patience = 0;
+                    if (tid == 0) fs_flag(&st->expired);
+                }
             }
             lds_barrier();
         }

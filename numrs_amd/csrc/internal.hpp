@@ -241,6 +241,8 @@ bool plan_is_fused(const Plan& p);
 // the last one are done (destroying a plan frees its workspace, which waits
 // for them).
 FsState* fs_state_take(DeviceCtx* ctx);
+// Waits for the stream; NRFFT_E_HIP if the word is set, and clears it.
+int expired_check(uint32_t* d_word, hipStream_t s);
 void fs_state_give(int device, FsState* st);
 int exec_launch(const Plan& p, const Launch& l, void* const* bufs, int isign, hipStream_t stream, DeviceCtx* ctx);
 int col_tilog(int dtype);

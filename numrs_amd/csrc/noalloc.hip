@@ -26,15 +26,15 @@
 #endif
 
 static __device__ __align__(256) unsigned char scratch[NRFFT_NOALLOC_SCRATCH_BYTES];
-// Counters of the fused launches (k_fused4), cleared before each: calls that
-// raced may have left them anyhow.
+// Counters of the fused launches (k_fused4), cleared before each (calls that
+// raced may have left them anyhow) up to `expired`, which the check clears.
 static __device__ nrfft::FsState fused_state;
 
 namespace nrfft {
 
 __global__ void k_fused_clear(FsState* st) {
-    uint32_t* p = reinterpret_cast<uint32_t*>(st);
-    for (unsigned i = threadIdx.x; i < sizeof(FsState) / 4; i += blockDim.x) p[i] = 0;
+    uint32_t* p = &st->ticket;
+    for (unsigned i = threadIdx.x; i < (sizeof(FsState) - offsetof(FsState, ticket)) / 4; i += blockDim.x) p[i] = 0;
 }
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -154,4 +154,13 @@ extern "C" int nrfft_execute_four1_batch_noalloc(int dtype, const void* d_in, vo
                                                  int isign, void* stream) {
     g_err.clear();
     return noalloc_c2c(dtype, d_in, d_out, nn, batch, isign, (hipStream_t)stream);
+}
+
+extern "C" int nrfft_four1_batch_noalloc_check(void* stream) {
+    g_err.clear();
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return fail(NRFFT_E_HIP, "hipGetDevice");
+    void *ws = nullptr, *state = nullptr;
+    if (int rc = scratch_of(dev, &ws, &state)) return rc;
+    return expired_check(&static_cast<FsState*>(state)->expired, (hipStream_t)stream);
 }

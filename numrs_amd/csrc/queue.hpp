@@ -53,8 +53,9 @@ struct QTask {
 };
 
 // Counters, each on a cache line of its own: tickets taken, groups that have
-// left, tickets taken in the last launch, then the slabs'.
-constexpr int Q_LINE = 32, Q_TICKET = 0, Q_DONE = 1, Q_LAST = 2, Q_SLABS = 3;
+// left, tickets taken in the last launch, whether a wait has given up (set until a
+// check reads it), then the slabs'.
+constexpr int Q_LINE = 32, Q_TICKET = 0, Q_DONE = 1, Q_LAST = 2, Q_EXPIRED = 3, Q_SLABS = 4;
 constexpr size_t Q_SLAB_TILES = 64, Q_PAIR_TILES = 640, Q_FEW_TILES = 768;
 
 // Stage-1 twiddles of all lengths: W_{n^2}^{r k} for k, r < n, n = 32 (FP32) and
@@ -262,7 +263,10 @@ k_queue(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, const QTask* __restrict__ t
                     if (__ballot(peek(q.wait, q.nwait) != 0) == 0) break;
                     __builtin_amdgcn_s_sleep(8);
                 }
-                if (i == patience) patience = 0;
+                if (i == patience) {
+                    patience = 0;
+                    if (tid == 0) fs_flag(line(Q_EXPIRED));
+                }
             }
             lds_barrier();
         }

@@ -32,6 +32,7 @@ struct UnevenState {
     int n1 = 0, n2 = 0;        // single- and first-pass tiles, second-pass tiles
     std::vector<uint32_t> offs;  // of the items of single-pass tiles, from their tile's base
     bool few = false;          // one group per CU
+    bool reused = false;       // parts of the ring are handed out more than once
     std::vector<uint32_t> init;  // the counters' initial values
     size_t ring_elems = 0;
     size_t total_elems = 0;
@@ -204,6 +205,7 @@ static int build_uneven(UnevenState& u, const std::vector<int>* force_split = nu
     for (const Two& t : two) total += t.work;
     const size_t ring = std::min(total, std::max<size_t>(4, FUSED_RING_BYTES / csize(u.dtype) / largest) * largest);
     u.ring_elems = ring;
+    u.reused = ring < total;
     // Slabs: consecutive items.
     const size_t tile = size_t(1) << qlog, slab_elems = Q_SLAB_TILES * tile;
     struct Slab {
@@ -605,6 +607,15 @@ int nrfft_uneven_check(nrfft_uneven plan, void* stream) {
     // every group leaves after drawing one ticket past the end
     if (2 * (uint64_t)tickets < (uint64_t)plan->u.tasks.size())
         return fail(NRFFT_E_HIP, "uneven queue: the task list was not drained");
+    return expired_check(plan->u.d_ctr + Q_EXPIRED * Q_LINE, (hipStream_t)stream);
+}
+
+int nrfft_uneven_launch_info(nrfft_uneven plan, int* launches, int* ring_reused, void** expired) {
+    g_err.clear();
+    if (!plan) return fail(NRFFT_E_INVALID, "null plan");
+    if (launches) *launches = 1;
+    if (ring_reused) *ring_reused = plan->u.reused ? 1 : 0;
+    if (expired) *expired = plan->u.d_ctr + Q_EXPIRED * Q_LINE;
     return NRFFT_OK;
 }
 

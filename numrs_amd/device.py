@@ -129,6 +129,20 @@ class _Plan:
     def num_launches(self) -> int:
         return int(_lib.lib().nrfft_plan_num_launches(self._h))
 
+    def check(self, stream=None) -> None:
+        """Wait for the stream; raise if a wait inside a launch of this plan has
+        given up since the last check (the results are then not valid)."""
+        _check(_lib.lib().nrfft_plan_check(self._h, _stream(stream)))
+
+    def launch_info(self, isign: int = 1) -> dict:
+        """What one execution enqueues: launches, and the slabs and ring slots of a
+        launch that runs several passes (0: none); expired: address of the word
+        that check() reads (None: no such launch)."""
+        n, slots, slabs, word = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p()
+        _check(_lib.lib().nrfft_plan_launch_info(self._h, isign, ctypes.byref(n), ctypes.byref(slots),
+                                                 ctypes.byref(slabs), ctypes.byref(word)))
+        return {"launches": n.value, "ring_slots": slots.value, "ring_slabs": slabs.value, "expired": word.value}
+
 
 class C2CPlan(_Plan):
     """Batched C2C of shape nn (C order); ndim 1 = four1, ndim >= 2 = fourn.
@@ -345,8 +359,15 @@ class UnevenPlan(_Plan):
         _check(fn(self._h, a, b, isign, _stream(stream)))
 
     def check(self, stream=None) -> None:
-        """Wait for the stream; raise if the last execution left tasks untaken."""
+        """Wait for the stream; raise if the last execution left tasks untaken or a
+        wait inside one has given up since the last check."""
         _check(_lib.lib().nrfft_uneven_check(self._h, _stream(stream)))
+
+    def launch_info(self, isign: int = 1) -> dict:
+        n, reused, word = ctypes.c_int(), ctypes.c_int(), ctypes.c_void_p()
+        _check(_lib.lib().nrfft_uneven_launch_info(self._h, ctypes.byref(n), ctypes.byref(reused),
+                                                   ctypes.byref(word)))
+        return {"launches": n.value, "ring_reused": bool(reused.value), "expired": word.value}
 
     def info(self) -> dict:
         a, b, w = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
