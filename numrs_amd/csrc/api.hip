@@ -103,7 +103,7 @@ int get_ctx(DeviceCtx** out) {
     hipLaunchKernelGGL(k_stage_twiddles, dim3(TW_STAGE_ELEMS / 256), dim3(256), 0, 0, c->c64s, c->c32s);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMalloc(&c->fs_pool, FS_POOL * sizeof(FsState)));
-    HIPCHK(hipMemset(c->fs_pool, 0, FS_POOL * sizeof(FsState)));
+    HIPCHK(hipStreamCreateWithFlags(&c->fs_stream, hipStreamNonBlocking));
     c->fs_free.reserve(FS_POOL);
     for (int i = FS_POOL; i-- > 0;) c->fs_free.push_back(c->fs_pool + i);
     if (int rc = build_mfma_tables(c)) return rc;
@@ -113,10 +113,18 @@ int get_ctx(DeviceCtx** out) {
     return NRFFT_OK;
 }
 
+static __global__ void k_state_zero(FsState* st) {
+    for (unsigned i = threadIdx.x; i < sizeof(FsState) / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(st)[i] = 0;
+}
 FsState* fs_state_take(DeviceCtx* ctx) {
     std::lock_guard<std::mutex> lk(g_ctx_mu);
     if (ctx->fs_free.empty()) return nullptr;
     FsState* st = ctx->fs_free.back();
+    hipLaunchKernelGGL(k_state_zero, dim3(1), dim3(256), 0, ctx->fs_stream, st);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->fs_stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     ctx->fs_free.pop_back();
     return st;
 }

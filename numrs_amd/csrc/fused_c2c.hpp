@@ -39,9 +39,10 @@
 // stays set until a check reads it (nrfft_plan_check).
 //
 // The last group to leave clears the counters, so a launch leaves the state
-// as it found it and needs no reset launch or memset before it.  (The count of
-// groups that have left is taken down by the launch's own: whatever overlapped,
-// the very last group finds the others gone and clears everything.)
+// as it found it and needs no reset launch or memset before it.  (Launches of one
+// plan have equal grids.  If some overlapped against the rules, the very last group
+// still brings the count of those that have left to a multiple of the grid, finds
+// it unchanged and clears everything; a plan takes a state that is cleared first.)
 #pragma once
 #include "pass_c2c.hpp"
 #include "real_fft.hpp"
@@ -424,6 +425,10 @@ __device__ __forceinline__ void fs_count(uint32_t* p) {
 }
 __device__ __forceinline__ void fs_flag(uint32_t* p) {
     __hip_atomic_store(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The count of groups that have left back to 0 unless more have left since.
+__device__ __forceinline__ void fs_all_left(uint32_t* done, uint32_t left) {
+    __hip_atomic_compare_exchange_strong(done, &left, 0u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Where a ring slot's tile is counted as loaded: the next tile's stores to the slot
 // may follow.  (The comment marks the place in the assembly, where
@@ -871,11 +876,12 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
     // the state (nobody reads it any more).
     fs_drain<0>();
     lds_barrier();
+    uint32_t left = 0;  // thread 0: groups that have left, this one included
     if (tid == 0) {
         if (pending) fs_count(pending);
         fs_drain<0>();
-        const uint32_t left = __hip_atomic_fetch_add(&st->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sh[0] = left == gridDim.x - 1;
+        left = __hip_atomic_fetch_add(&st->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+        sh[0] = left % gridDim.x == 0;
     }
     lds_barrier();
     if (sh[0]) {
@@ -885,7 +891,7 @@ k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twi
         }
         if (tid == 0) {
             __hip_atomic_store(&st->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_sub(&st->done, gridDim.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            fs_all_left(&st->done, left);
         }
     }
 }

@@ -32,8 +32,9 @@ struct DeviceCtx {
     c32* c32f = nullptr;
     c64* c64s = nullptr;  // per-stage tables (TW_STAGE_ELEMS entries)
     c32* c32s = nullptr;
-    FsState* fs_pool = nullptr;     // FS_POOL counter blocks of fused plans, zeroed
+    FsState* fs_pool = nullptr;     // FS_POOL counter blocks of fused plans
     std::vector<FsState*> fs_free;  // those no plan holds (guarded by the context lock)
+    hipStream_t fs_stream = nullptr;  // where they are cleared: no caller's stream, not ordered with any
     void* mfma_f16 = nullptr;   // split-precision DFT-matrix operands
     void* mfma_bf16 = nullptr;
     int ncu = 256;        // compute units
@@ -235,11 +236,10 @@ inline int64_t fused_min_tiles(bool f32, int logn, int form) {
 }
 constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;
 bool plan_is_fused(const Plan& p);
-// A zeroed FsState of the current device's pool for a plan with fused
-// launches (nullptr: none left), and its return.  A launch leaves its counters
-// zero, so a returned state is ready for the next plan once the launches of
-// the last one are done (destroying a plan frees its workspace, which waits
-// for them).
+// A FsState of the current device's pool for a plan with fused launches (nullptr:
+// none left), cleared whatever its last plan left in it, and its return (when that
+// plan's launches are done: destroying a plan frees its workspace, which waits for
+// them).
 FsState* fs_state_take(DeviceCtx* ctx);
 // Waits for the stream; NRFFT_E_HIP if the word is set, and clears it.
 int expired_check(uint32_t* d_word, hipStream_t s);

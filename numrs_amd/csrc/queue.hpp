@@ -300,17 +300,19 @@ k_queue(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, const QTask* __restrict__ t
     // Leave; the last group sets the counters for the next launch.
     fs_drain<0>();
     lds_barrier();
+    uint32_t left = 0;  // (as k_fused4)
     if (tid == 0) {
         if (pending) q_count(pending);
         fs_drain<0>();
-        sh[0] = __hip_atomic_fetch_add(line(Q_DONE), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        left = __hip_atomic_fetch_add(line(Q_DONE), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+        sh[0] = left % gridDim.x == 0;
     }
     lds_barrier();
     if (sh[0]) {
         if (tid == 0) {
             __hip_atomic_store(line(Q_LAST), fs_peek(line(Q_TICKET)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(line(Q_TICKET), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_sub(line(Q_DONE), gridDim.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            fs_all_left(line(Q_DONE), left);
         }
         for (int i = Q_SLABS + tid; i < lines; i += FS_NT)
             __hip_atomic_store(line(i), init[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
