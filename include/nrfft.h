@@ -217,8 +217,8 @@ int nrfft_execute_rlft3(nrfft_plan plan, void* d_data, void* d_speq, int isign, 
 
 /* ---- uneven batches -------------------------------------------------------
  * Many transforms of different lengths and dimensionality in one persistent
- * work-queue kernel (two dispatches, one per pass phase, replayed as a
- * captured hipGraph).  Item i has ndim[i] (1 or 2) and dims dims[2 i]
+ * work-queue kernel (or one launch per pass, where that is faster or memory is
+ * short), replayed as a captured hipGraph.  Item i has ndim[i] (1 or 2) and dims dims[2 i]
  * (, dims[2 i + 1]) in C order, powers of two >= 64 (2-D sides up to 8192 in
  * FP32 / 4096 in FP64; 1-D up to 2^24 in FP32 / 2^22 in FP64), and lives at
  * complex-element offset offs[i] of both d_in and d_out (in place allowed).

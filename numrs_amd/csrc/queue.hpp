@@ -23,7 +23,8 @@
 // memory side.  500 items of mixed shapes, FP32 (914 MB): 583 us; as two launches,
 // one a pass with the whole intermediate in memory, 840 (HBM traffic twice).
 // 16 of 2048 x 2048 390 us against 575 (second-pass tiles of eight columns write
-// 64-byte runs), 64 of 1024 x 1024 335 against 525, 8 small items as before.
+// 64-byte runs), 64 of 1024 x 1024 335 against 525.  Batches that are faster as two
+// launches (few tiles of long passes): queue_passes.hpp.
 //
 // In the ring an item lies in blocks [second-pass tile][first-pass tile][kk][t]
 // (kk: transform of the second-pass tile, t: of the first), so that a tile of
@@ -115,7 +116,11 @@ __device__ __forceinline__ void q_tile(const QTask& q, const cpx<T>* in, cpx<T>*
         using E = QEng<T, S, LOGL, MODE>;
         constexpr int EPT = E::EPT;
         constexpr int AUX_IN = MODE == Q_RING ? FS_AUX_SC1 : FS_AUX_NT;
-        constexpr int AUX_OUT = MODE == Q_ROW || MODE == Q_RING ? FS_AUX_NT : FS_AUX_SC1;
+        // Results are not read again (NT), but runs of less than 64 bytes (sides of 4096
+        // and 8192) have to meet their line's other runs in the L2 first: 4096 x 4096 FP32
+        // 228 us against 388, 8 of 2048 x 2048 (64-byte runs) 242 against 221 with NT.
+        constexpr int AUX_OUT = MODE == Q_COL || MODE == Q_ROWS ? FS_AUX_SC1
+                                : MODE == Q_RING && E::TI * CS < 64 ? 0 : FS_AUX_NT;
         // A transform that does not exist is out of its buffer's range: loads
         // give 0, stores are dropped.  (Four-step tiles are always full.)
         auto valid = [&](uint32_t off, int t) {

@@ -10,6 +10,7 @@
 #include "../../include/nrfft.h"
 #include "internal.hpp"
 #include "queue.hpp"
+#include "uneven.hpp"
 
 namespace nrfft {
 
@@ -19,19 +20,15 @@ namespace nrfft {
         if (e_ != hipSuccess) return fail(NRFFT_E_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-struct UnevenItem {
-    int ndim;
-    size_t n0, n1;  // ndim == 1: n0 = N, n1 = 1
-    size_t off;     // complex elements
-};
-
 struct UnevenState {
     int dtype = 0;
     std::vector<UnevenItem> items;
+    std::unique_ptr<UnevenPasses> passes;  // one launch a pass; the list below is then not used
     std::vector<QTask> tasks;  // in the order in which they are taken, two to a ticket
     int n1 = 0, n2 = 0;        // single- and first-pass tiles, second-pass tiles
     std::vector<uint32_t> offs;  // of the items of single-pass tiles, from their tile's base
     bool few = false;          // one group per CU
+    bool slow_list = false;    // faster with one launch a pass
     bool reused = false;       // parts of the ring are handed out more than once
     std::vector<uint32_t> init;  // the counters' initial values
     size_t ring_elems = 0;
@@ -54,11 +51,16 @@ struct UnevenState {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         if (cap) (void)hipStreamDestroy(cap);
-        if (d_tasks) (void)hipFree(d_tasks);
-        if (d_offs) (void)hipFree(d_offs);
-        if (d_init) (void)hipFree(d_init);
-        if (d_ctr) (void)hipFree(d_ctr);
-        if (d_ring) (void)hipFree(d_ring);
+        drop_list();
+    }
+    void drop_list() {
+        for (void* p : {(void*)d_tasks, (void*)d_offs, (void*)d_init, (void*)d_ctr, d_ring})
+            if (p) (void)hipFree(p);
+        d_tasks = nullptr;
+        d_offs = d_init = d_ctr = nullptr;
+        d_ring = nullptr;
+        tasks = {};
+        offs = init = {};
     }
 };
 
@@ -146,12 +148,46 @@ static std::vector<QTask> single_tiles(int dtype, const std::vector<std::pair<in
 
 // Four-step split of a 1-D item of 2^logn points: the autotuned choice for
 // its size class when the tune cache holds one, else N1 = 2^floor(logn / 2).
-static int uneven_split(int dtype, int logn, int lo, int hi, const std::vector<int>* force) {
+int uneven_split(int dtype, int logn, int lo, int hi, const std::vector<int>* force) {
     if (force && (size_t)logn < force->size() && (*force)[logn] > 0) return (*force)[logn];
     Tune t;
     if (tune_find(PK_UNEVEN, dtype, {size_t(1) << logn}, 0, &t) && t.split_log1 >= lo && t.split_log1 <= hi)
         return t.split_log1;
     return std::min(hi, std::max(lo, logn / 2));
+}
+
+// Whether an item of two passes of 2^la and 2^lb points runs faster with one launch
+// a pass, in a batch of `tiles` first-pass tiles.  A tile of three or four stages
+// (2048 points and more) takes longer in the list's engine, which shows while the
+// tiles are few; 8192-point passes and the 32-byte runs of a 4096 x 4096 item's
+// columns lose at any number.  Batches of one shape, MI355X, one launch a pass / list
+// (us):
+//   FP32 1 of 2^21 41 / 48, 2: 47 / 56, 4: 75 / 73; 1 of 2^22 49 / 71, 2: 81 / 85,
+//   4: 167 / 142; 1 of 2048 x 2048 50 / 64, 2: 83 / 73; 2 of 1024 x 2048 48 / 54, 4: 76 / 70;
+//   1 of 4096 x 4096 172 / 230, 2: 386 / 433; 1 of 256 x 8192 42 / 49, 8: 129 / 145, 16:
+//   267 / 265; 1 of 8192 x 256 58 / 61, of 8192 x 2048 244 / 387; 1 of 2^20 36 / 33, of
+//   1024 x 1024 38 / 32.
+//   FP64 1 of 2^20 41 / 41, 2: 46 / 55, 4: 73 / 66; 1 of 2^22 82 / 106, 2: 175 / 157;
+//   8 of 2^18 45 / 49, 16: 72 / 62; 1 of 4096 x 4096 381 / 509, of 4096 x 2048 170 / 211.
+static bool item_faster_in_passes(bool f32, int la, int lb, bool cols, size_t tiles) {
+    const int s = la + lb, longest = std::max(la, lb);
+    if (s >= 24) return true;
+    if (f32) {
+        if (longest == 13) return tiles <= 2048;
+        if (s == 23) return tiles <= (cols ? 640 : 512);
+        if (s == 22) return tiles <= (cols ? 640 : 256);
+        return s == 21 && tiles <= 256 && (cols || tiles > 128);
+    }
+    if (!cols && lb == 12 && la >= 10) return true;
+    if (s == 23) return tiles <= 1024;
+    if (s == 22) return tiles <= (longest == 13 ? 1024 : 896);
+    if (tiles > 256) return false;
+    return s == 21 || longest == 13 || (s >= 18 && tiles > 128 && lb <= 10);
+}
+// Likewise for single-pass items: only 8192-point ones (FP64 256 of them 31 / 43 us,
+// 100: 26 / 24, 800: 70 / 69; FP32 16 23 / 24, as plain launches 15 / 19, 256 28 / 26).
+static bool row_faster_in_passes(bool f32, int logn, size_t tiles) {
+    return logn == 13 && (f32 ? tiles <= 64 : tiles > 128 && tiles < 700);
 }
 
 // The list of tiles (queue.hpp): items largest first, collected into slabs of
@@ -265,6 +301,17 @@ static int build_uneven(UnevenState& u, const std::vector<int>* force_split = nu
         u.n2 += (int)s.b.size();
         if (s.w1 - s.w0 > 64) return fail(NRFFT_E_UNSUPPORTED, "uneven ring order");
     }
+    // One launch a pass if that is faster for most of the work.
+    size_t points = 0, slow = 0;
+    for (const Two& t : two) {
+        points += t.work;
+        if (item_faster_in_passes(f32, t.p.la, t.p.lb, t.p.cols, (size_t)u.n1)) slow += t.work;
+    }
+    for (const auto& o : one) {
+        points += size_t(1) << o.first;
+        if (row_faster_in_passes(f32, o.first, (size_t)u.n1)) slow += size_t(1) << o.first;
+    }
+    u.slow_list = 2 * slow > points;
     if ((size_t)u.n1 + (size_t)u.n2 > size_t(1) << 30) return fail(NRFFT_E_UNSUPPORTED, "uneven batch of too many tiles");
 
     // Few tiles: one group per CU, so that they spread over the chip (720 first-pass
@@ -333,7 +380,11 @@ static int uneven_setup_device(UnevenState& u) {
     HIPCHK(hipMemcpy(u.d_ctr, ctr.data(), ctr.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     if (u.ring_elems) {
         const size_t bytes = u.ring_elems * csize(u.dtype);
-        if (hipMalloc(&u.d_ring, bytes) != hipSuccess) return fail(NRFFT_E_NOMEM, "uneven workspace");
+        if (hipMalloc(&u.d_ring, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            u.d_ring = nullptr;
+            return fail(NRFFT_E_NOMEM, "uneven workspace");
+        }
     }
     for (int d = 0; d < 2; ++d) {
         const void* fn = u.dtype == NRFFT_F32 ? queue_kernel<float>(d == 0 ? 1 : -1)
@@ -343,12 +394,32 @@ static int uneven_setup_device(UnevenState& u) {
         if (per_cu < 1) return fail(NRFFT_E_UNSUPPORTED, "queue kernel does not fit a CU");
         u.grid[d] = (unsigned)((u.few ? 1 : per_cu) * ctx->ncu);
     }
+    return NRFFT_OK;
+}
+
+// The plan's launches: one list, or one launch a pass where that is faster or the
+// ring finds no room.
+static int uneven_make(UnevenState& u, const std::vector<int>* force_split = nullptr) {
+    int rc = build_uneven(u, force_split);
+    if (rc) return rc;
+    bool passes = u.slow_list;
+    if (!passes) {
+        rc = uneven_setup_device(u);
+        passes = rc == NRFFT_E_NOMEM;
+        if (rc && !passes) return rc;
+    }
+    if (passes) {
+        u.drop_list();
+        u.passes = std::make_unique<UnevenPasses>();
+        if ((rc = u.passes->build(u.dtype, u.items, force_split)) || (rc = u.passes->setup_device())) return rc;
+    }
     HIPCHK(hipStreamCreateWithFlags(&u.cap, hipStreamNonBlocking));
     return NRFFT_OK;
 }
 
 template <typename T>
 static int uneven_enqueue(UnevenState& u, const void* in, void* out, int isign, hipStream_t s) {
+    if (u.passes) return u.passes->enqueue(in, out, isign, s);
     DeviceCtx* ctx = nullptr;
     int rc = get_ctx(&ctx);
     if (rc) return rc;
@@ -464,8 +535,7 @@ static int autotune_uneven(int dtype, int lmin, int lmax, int iters, int* best_l
             u.total_elems = count * n;
             std::vector<int> force(size_t(logn) + 1, 0);
             force[logn] = l1;
-            int rc = build_uneven(u, &force);
-            if (!rc) rc = uneven_setup_device(u);
+            int rc = uneven_make(u, &force);
             float ms = 0.f;
             if (!rc) rc = f32 ? time_uneven<float>(u, r.in, r.out, iters, r.s, r.e0, r.e1, &ms)
                               : time_uneven<double>(u, r.in, r.out, iters, r.s, r.e0, r.e1, &ms);
@@ -574,9 +644,7 @@ int nrfft_plan_uneven(nrfft_uneven* plan, int dtype, size_t nitems, const int* n
         p->u.items.push_back(it);
     }
     p->u.total_elems = end;
-    int rc = build_uneven(p->u);
-    if (rc) return rc;
-    rc = uneven_setup_device(p->u);
+    int rc = uneven_make(p->u);
     if (rc) return rc;
     *plan = p.release();
     return NRFFT_OK;
@@ -601,6 +669,7 @@ int nrfft_execute_uneven_nograph(nrfft_uneven plan, const void* d_in, void* d_ou
 int nrfft_uneven_check(nrfft_uneven plan, void* stream) {
     g_err.clear();
     if (!plan) return fail(NRFFT_E_INVALID, "null plan");
+    if (plan->u.passes) return plan->u.passes->check((hipStream_t)stream);
     uint32_t tickets = 0;
     HIPCHK(hipMemcpyAsync(&tickets, plan->u.d_ctr + Q_LAST * Q_LINE, sizeof tickets, hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
@@ -613,9 +682,10 @@ int nrfft_uneven_check(nrfft_uneven plan, void* stream) {
 int nrfft_uneven_launch_info(nrfft_uneven plan, int* launches, int* ring_reused, void** expired) {
     g_err.clear();
     if (!plan) return fail(NRFFT_E_INVALID, "null plan");
-    if (launches) *launches = 1;
-    if (ring_reused) *ring_reused = plan->u.reused ? 1 : 0;
-    if (expired) *expired = plan->u.d_ctr + Q_EXPIRED * Q_LINE;
+    const UnevenState& u = plan->u;
+    if (launches) *launches = u.passes ? u.passes->launches() : 1;
+    if (ring_reused) *ring_reused = !u.passes && u.reused ? 1 : 0;
+    if (expired) *expired = u.passes ? nullptr : u.d_ctr + Q_EXPIRED * Q_LINE;
     return NRFFT_OK;
 }
 
@@ -623,10 +693,11 @@ int nrfft_uneven_info(nrfft_uneven plan, size_t* tasks_phase1, size_t* tasks_pha
                       unsigned* groups) {
     g_err.clear();
     if (!plan) return fail(NRFFT_E_INVALID, "null plan");
-    if (tasks_phase1) *tasks_phase1 = (size_t)plan->u.n1;
-    if (tasks_phase2) *tasks_phase2 = (size_t)plan->u.n2;
-    if (workspace_bytes) *workspace_bytes = plan->u.ring_elems * csize(plan->u.dtype);
-    if (groups) *groups = plan->u.grid[0];
+    const UnevenState& u = plan->u;
+    if (tasks_phase1) *tasks_phase1 = (size_t)(u.passes ? u.passes->n1 : u.n1);
+    if (tasks_phase2) *tasks_phase2 = (size_t)(u.passes ? u.passes->n2 : u.n2);
+    if (workspace_bytes) *workspace_bytes = (u.passes ? u.passes->ws_elems : u.ring_elems) * csize(u.dtype);
+    if (groups) *groups = u.passes ? u.passes->grid[0] : u.grid[0];
     return NRFFT_OK;
 }
 
