@@ -68,6 +68,17 @@ static int scratch_of(int device, void** out, void** state) {
     return NRFFT_OK;
 }
 
+// Fewest tiles of a pass for the fused launch with the 64 MiB ring, whose places are
+// used again after 512 tiles and which feeds one group a CU.  MI355X, separate passes /
+// fused (us): FP32 2^15 768 tiles 78 / 89, 1280 130 / 134, 1536 154 / 147; 2^18 1024
+// 108 / 111, 1152 129 / 120; 2^19 768 90 / 96, 896 108 / 100; 2^20 640 85 / 78; 2^21 (16
+// MiB a slab) 768 95 / 119, 2048 246 / 247, 2944 362 / 341; FP64 2^16 768 77 / 86, 1024
+// 100 / 101, 1152 118 / 112; 2^20 1280 149 / 154, 1664 198 / 188.
+static int64_t noalloc_min_tiles(bool f32, int logn) {
+    if (!f32) return logn == 20 ? 1664 : 1152;
+    return logn == 21 ? 2944 : logn == 20 ? 640 : logn == 19 ? 896 : logn == 18 ? 1152 : 1536;
+}
+
 static int noalloc_c2c(int dtype, const void* d_in, void* d_out, size_t nn, size_t batch, int isign,
                        hipStream_t stream) {
     if (dtype != NRFFT_F32 && dtype != NRFFT_F64) return fail(NRFFT_E_INVALID, "dtype");
@@ -120,7 +131,8 @@ static int noalloc_c2c(int dtype, const void* d_in, void* d_out, size_t nn, size
     }
     Launch fused;
     size_t ring = 0;
-    if (fused_launch(p, logn, (int64_t)batch, B_IN, B_OUT, NRFFT_NOALLOC_SCRATCH_BYTES, &fused, &ring)) {
+    if (fused_launch(p, logn, (int64_t)batch, B_IN, B_OUT, NRFFT_NOALLOC_SCRATCH_BYTES, &fused, &ring, FUSED_C2C,
+                     noalloc_min_tiles(dtype == NRFFT_F32, logn))) {
         hipLaunchKernelGGL(k_fused_clear, dim3(1), dim3(256), 0, stream, (FsState*)state);
         if (hipGetLastError() != hipSuccess) return fail(NRFFT_E_HIP, "k_fused_clear");
         return exec_launch(p, fused, bufs, isign, stream, ctx);
