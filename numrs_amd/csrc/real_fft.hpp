@@ -375,10 +375,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(conv_waves<T
     //   Ye = Xe Re + W_L^p Xo Ro,         Yo = Xe Ro + Xo Re          (convolution)
     //   Ye = Xe Re* + Xo Ro*,             Yo = Xo Re* + W_L^-p Xe Ro* (correlation)
     // and the pair of the inverse's input Ye + i Yo, conj(Ye - i Yo): 40
-    // instructions a pair instead of 68 (4096 x 2^14, 257 taps: 250 us against 253; 2^15, full FFTs, 337 against 351).
+    // instructions a pair instead of 68 (FP32 4096 x 2^14, 257 taps: 252 us against 253; 2048 x
+    // 2^15, full FFTs, 344 against 355; FP64 4096 x 2^13 241 against 246).
+    // (The 1 / (n / 2) goes onto the product: on one operand it would take values
+    // below 2^-110 out of the 32-bit range.)
     auto split = [](cpx<T> a, cpx<T> b, T f, cpx<T>& e, cpx<T>& o) {
-        e = cpx<T>{f * a.x + f * b.x, f * a.y - f * b.y};
-        o = cpx<T>{f * a.y + f * b.y, f * b.x - f * a.x};
+        e = cpx<T>{f * (a.x + b.x), f * (a.y - b.y)};
+        o = cpx<T>{f * (a.y + b.y), f * (b.x - a.x)};
     };
 
     // The two forward transforms share the tile: the first one's spectrum is
@@ -438,7 +441,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(conv_waves<T
             ha[u] = dc_forward(lds[hidx(t, 0)]);
             hb[u] = lds[hidx(t, NP)];
         } else if (halves) {
-            split(lds[hidx(t, p)], lds[hidx(t, L - p)], (T)0.25 * inv_no2, ha[u], hb[u]);
+            split(lds[hidx(t, p)], lds[hidx(t, L - p)], (T)0.5, ha[u], hb[u]);
         } else {
             untangle_pair(lds[hidx(t, p)], lds[hidx(t, L - p)], wpair(u), (T)-0.5, ha[u], hb[u]);
         }
@@ -468,7 +471,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(conv_waves<T
             lds[EF::lidx(t, NP)] = spec_apply(op, xh, rh, inv_no2);
         } else if (halves) {
             cpx<T> xe, xo, ye, yo;
-            split(lds[EF::lidx(t, p)], lds[EF::lidx(t, L - p)], (T)1, xe, xo);
+            split(lds[EF::lidx(t, p)], lds[EF::lidx(t, L - p)], (T)1, xe, xo);  // 2 Xe, 2 Xo
             const cpx<T> re = ha[u], ro = hb[u], w = wpair(u);
             if (op == OP_CONV) {
                 ye = cmul(xe, re) + cmul(xo, cmul(w, ro));
@@ -477,8 +480,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(conv_waves<T
                 ye = cmulc(xe, re) + cmulc(xo, ro);
                 yo = cmulc(xo, re) + cmulc(xe, cmul(w, ro));
             }
-            lds[EF::lidx(t, p)] = cpx<T>{ye.x - yo.y, ye.y + yo.x};
-            lds[EF::lidx(t, L - p)] = cpx<T>{ye.x + yo.y, yo.x - ye.y};
+            lds[EF::lidx(t, p)] = cscale(cpx<T>{ye.x - yo.y, ye.y + yo.x}, (T)0.5 * inv_no2);
+            lds[EF::lidx(t, L - p)] = cscale(cpx<T>{ye.x + yo.y, yo.x - ye.y}, (T)0.5 * inv_no2);
         } else {
             cpx<T> ta, tb, oa, ob2;
             const cpx<T> w = wpair(u);
