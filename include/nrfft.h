@@ -53,6 +53,11 @@ const char* nrfft_last_error(void);
 /* Select the HIP device used by this thread and build its twiddle tables
  * (FP64, generated on the GPU).  Optional: every call initialises lazily. */
 int nrfft_init(int device);
+/* Gives back the device and pinned memory that host-pointer calls keep for the next
+ * one on the current device (up to four blocks of 1 to 32 MiB and 2 MiB of pinned
+ * memory each); blocks of calls that are running stay.  Happens by itself when a plan
+ * or call finds no room. */
+int nrfft_trim(void);
 
 /* ---- 1. host-pointer drop-in calls ------------------------------------- */
 

@@ -44,6 +44,7 @@ _SIGS = {
     "nrfft_status_string": (ctypes.c_char_p, [_i]),
     "nrfft_last_error": (ctypes.c_char_p, []),
     "nrfft_init": (_i, [_i]),
+    "nrfft_trim": (_i, []),
     "nrfft_four1_f64": (_i, [_dp, _sz, _i]),
     "nrfft_four1_f32": (_i, [_fp, _sz, _i]),
     "nrfft_four1_batch_f64": (_i, [_dp, _sz, _sz, _i]),

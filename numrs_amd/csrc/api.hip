@@ -934,10 +934,27 @@ int build_plan(Plan& p) {
     }
 }
 
+hipError_t dev_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && lanes_trim()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 int dev_alloc(DevBuf& b, size_t bytes, hipStream_t s) {
     b.s = s;
     if (bytes == 0) return NRFFT_OK;
     hipError_t e = hipMallocAsync(&b.p, bytes, s);
+    if (e != hipSuccess && lanes_trim()) {
+        (void)hipGetLastError();
+        e = hipMallocAsync(&b.p, bytes, s);
+    }
     if (e != hipSuccess) {
         b.p = nullptr;
         return fail(NRFFT_E_NOMEM, std::string("hipMallocAsync: ") + hipGetErrorString(e));
@@ -1011,7 +1028,7 @@ int make_plan(nrfft_plan* plan, int kind, int dtype, std::vector<size_t> nn, siz
     }
     if (!rc && p->plan.tmp_elems) {
         size_t bytes = p->plan.tmp_elems * csize(dtype);
-        e = hipMalloc(&p->tmp, bytes);
+        e = dev_malloc(&p->tmp, bytes);
         if (e != hipSuccess && p->plan.fs_state) {
             // No room for the ring of the fused launches.
             (void)hipGetLastError();
@@ -1020,7 +1037,7 @@ int make_plan(nrfft_plan* plan, int kind, int dtype, std::vector<size_t> nn, siz
             rc = unfused();
             if (!rc) {
                 bytes = p->plan.tmp_elems * csize(dtype);
-                e = bytes ? hipMalloc(&p->tmp, bytes) : hipSuccess;
+                e = bytes ? dev_malloc(&p->tmp, bytes) : hipSuccess;
             }
         }
         if (!rc && e != hipSuccess && kind == PK_C2C && p->plan.nn.size() > 1 && !p->plan.strided_one_pass) {
@@ -1035,7 +1052,7 @@ int make_plan(nrfft_plan* plan, int kind, int dtype, std::vector<size_t> nn, siz
             if (!rc) {
                 p->plan = std::move(q);
                 bytes = p->plan.tmp_elems * csize(dtype);
-                e = bytes ? hipMalloc(&p->tmp, bytes) : hipSuccess;
+                e = bytes ? dev_malloc(&p->tmp, bytes) : hipSuccess;
             }
         }
         if (rc) {
@@ -1199,6 +1216,12 @@ int nrfft_plan_destroy(nrfft_plan plan) {
 size_t nrfft_plan_workspace_bytes(nrfft_plan plan) { return plan ? plan->tmp_bytes : 0; }
 
 int nrfft_plan_num_launches(nrfft_plan plan) { return plan ? (int)plan->plan.launches.size() : 0; }
+
+int nrfft_trim(void) {
+    g_err.clear();
+    (void)lanes_trim();
+    return NRFFT_OK;
+}
 
 int nrfft_plan_check(nrfft_plan plan, void* stream) {
     g_err.clear();

@@ -224,6 +224,25 @@ HostLane* lane_take(size_t bytes) {
     return best;
 }
 
+}  // namespace
+
+size_t lanes_trim() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    std::lock_guard<std::mutex> lk(g_lane_mu);
+    size_t freed = 0;
+    for (HostLane& l : g_lanes[dev]) {
+        if (l.busy) continue;  // (an idle lane's last call has waited for its stream)
+        if (l.d) (void)hipFree(l.d);
+        if (l.pin) (void)hipHostFree(l.pin);
+        freed += l.cap;
+        l = HostLane{};
+    }
+    return freed;
+}
+
+namespace {
+
 struct CopySegs {
     const uint4* src[4];
     uint4* dst[4];

@@ -260,14 +260,19 @@ struct DevBuf {
     }
 };
 int dev_alloc(DevBuf& b, size_t bytes, hipStream_t s);
+// hipMalloc, once more without the idle lanes of the host-pointer calls if there is
+// no room (*p: nullptr then).
+hipError_t dev_malloc(void** p, size_t bytes);
 // Device memory and transfers of one host-pointer call on stream s: open() with
 // the bytes of all its buffers, alloc() them, upload(), run, download(),
 // finish().  Calls of up to HOST_LANE_MAX bytes borrow a lane (a device block and
-// pinned staging, at most HOST_LANES a device, kept by the process); others, and
-// calls that find no lane free, allocate on the stream.
+// pinned staging, at most HOST_LANES a device); others, and calls that find no lane
+// free, allocate on the stream.  Lanes keep their memory until lanes_trim.
 constexpr size_t HOST_LANE_MAX = size_t(32) << 20;
 constexpr int HOST_LANES = 4;
 struct HostLane;
+// Frees the current device's lanes that no call holds; bytes of device memory freed.
+size_t lanes_trim();
 struct HostCall {
     explicit HostCall(hipStream_t st) : s(st) {}
     ~HostCall();

@@ -380,11 +380,7 @@ static int uneven_setup_device(UnevenState& u) {
     HIPCHK(hipMemcpy(u.d_ctr, ctr.data(), ctr.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     if (u.ring_elems) {
         const size_t bytes = u.ring_elems * csize(u.dtype);
-        if (hipMalloc(&u.d_ring, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            u.d_ring = nullptr;
-            return fail(NRFFT_E_NOMEM, "uneven workspace");
-        }
+        if (dev_malloc(&u.d_ring, bytes) != hipSuccess) return fail(NRFFT_E_NOMEM, "uneven workspace");
     }
     for (int d = 0; d < 2; ++d) {
         const void* fn = u.dtype == NRFFT_F32 ? queue_kernel<float>(d == 0 ? 1 : -1)

@@ -114,11 +114,8 @@ int UnevenPasses::setup_device() {
     HIPCHK(hipMalloc(&d_tasks, std::max<size_t>(1, tasks.size()) * sizeof(QPass)));
     if (!tasks.empty()) HIPCHK(hipMemcpy(d_tasks, tasks.data(), tasks.size() * sizeof(QPass), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&d_state, sizeof(QPState)));
-    if (ws_elems && hipMalloc(&d_ws, ws_elems * csize(dtype)) != hipSuccess) {
-        (void)hipGetLastError();
-        d_ws = nullptr;
+    if (ws_elems && dev_malloc(&d_ws, ws_elems * csize(dtype)) != hipSuccess)
         return fail(NRFFT_E_NOMEM, "uneven workspace");
-    }
     for (int d = 0; d < 2; ++d) {
         const void* fn = dtype == NRFFT_F32 ? pass_kernel<float>(d == 0 ? 1 : -1) : pass_kernel<double>(d == 0 ? 1 : -1);
         const int nt = dtype == NRFFT_F32 ? qp_pts<float>() / 16 : qp_pts<double>() / 16;
