@@ -186,8 +186,9 @@ __global__ __launch_bounds__(NT) void k_cosft1(const T* y, T* out, int64_t nsig,
     const T* yb = y + s0 * S;
     if constexpr (LTM > 0) E::template stage_tw_to_lds<LTM>(ltw, tw.stage, tid);  // read after the first exchange
     // Bin pairs (p, L - p), p < L / 2; the thread of p = 0 takes the bins 0 and L / 2.
-    constexpr int NP = L / 2;
-    constexpr int PPT1 = (TI * NP + NT - 1) / NT;
+    // (FP64 n = 8: L / 2 + 1 pairs, the last with itself; 2^22 signals 167 us against 170.)
+    constexpr int NP = L / 2, NPF = sizeof(T) == 8 && L == 8 ? NP + 1 : NP;
+    constexpr int PPT1 = (TI * NPF + NT - 1) / NT;
     __shared__ cpx<T> uw[PPT1];
     PairTw<T, PPT1> ptw;
     if constexpr (TI == 1) ptw.init(uw, tw, tid, NT, LOG2N2);
@@ -255,21 +256,21 @@ __global__ __launch_bounds__(NT) void k_cosft1(const T* y, T* out, int64_t nsig,
 #pragma unroll
     for (int u = 0; u < PPT1; ++u) {
         const int q = tid + u * NT;
-        if ((TI * NP) % NT != 0 && q >= TI * NP) break;
-        const int t = TI == 1 ? 0 : q / NP, p = TI == 1 ? q : q % NP;
+        if ((TI * NPF) % NT != 0 && q >= TI * NPF) break;
+        const int t = TI == 1 ? 0 : q / NPF, p = TI == 1 ? q : q % NPF;
         if (TI > 1 && t >= nvalid) continue;
         T* os = out + (s0 + t) * S;
         if (p == 0) {
             const cpx<T> z0 = lds[E::lidx(t, 0)];
             os[0] = half * (z0.x + z0.y);
             os[L] = half * (z0.x - z0.y);
-            os[NP] = half * lds[E::lidx(t, NP)].x;
+            if (NPF == NP) os[NP] = half * lds[E::lidx(t, NP)].x;
         } else {
             cpx<T> fa, fb;
             const cpx<T> w = TI == 1 ? ptw.at(uw, u) : twiddle_big<1>(tw, (uint32_t)p, LOG2N2);
             untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], w, (T)-0.5, fa, fb);
             os[p] = half * fa.x;
-            os[L - p] = half * fb.x;
+            if (NPF == NP || L - p != p) os[L - p] = half * fb.x;
         }
     }
 }
@@ -314,18 +315,20 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
             const T* ys = yb + t * N;
             return cpx<T>{ys[cf2_pos(2 * m, L)], ys[cf2_pos(2 * m + 1, L)]};
         }, false, ltw);
+        // (FP64 n = 16: L / 2 + 1 pairs, the last with itself; 2^20 signals 94 us against 96.)
+        constexpr int NPF = sizeof(T) == 8 && L == 8 ? NP + 1 : NP, PPTF = (TI * NPF + NT - 1) / NT;
 #pragma unroll
-        for (int u = 0; u < PPT2; ++u) {
+        for (int u = 0; u < PPTF; ++u) {
             const int q = tid + u * NT;
-            if ((TI * NP) % NT != 0 && q >= TI * NP) break;
-            const int t = TI == 1 ? 0 : q / NP, p = TI == 1 ? q : q % NP;
+            if ((TI * NPF) % NT != 0 && q >= TI * NPF) break;
+            const int t = TI == 1 ? 0 : q / NPF, p = TI == 1 ? q : q % NPF;
             if (TI > 1 && t >= nvalid) continue;
             T* os = out + (s0 + t) * N;
             if (p == 0) {
                 const cpx<T> z0 = lds[E::lidx(t, 0)];
                 os[0] = z0.x + z0.y;
                 os[L] = (z0.x - z0.y) * cos_quarter_pi<T>();
-                cf2_fwd_out_w(w16, lds[E::lidx(t, NP)], NP, os, N);
+                if (NPF == NP) cf2_fwd_out_w(w16, lds[E::lidx(t, NP)], NP, os, N);
             } else if constexpr (TI == 1) {
                 cpx<T> va, vb;
                 untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], pn.at(uwn, u), (T)-0.5, va, vb);
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(NT) void k_cosft2(const T* y, T* out, int64_t nsig,
                 untangle_pair(lds[E::lidx(t, p)], lds[E::lidx(t, L - p)], twiddle_big<1>(tw, (uint32_t)p, LOGN),
                               (T)-0.5, va, vb);
                 cf2_fwd_out(tw, va, p, LOGN, os, N);
-                cf2_fwd_out(tw, vb, L - p, LOGN, os, N);
+                if (NPF == NP || L - p != p) cf2_fwd_out(tw, vb, L - p, LOGN, os, N);
             }
         }
     } else {
