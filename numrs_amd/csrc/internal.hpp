@@ -230,8 +230,10 @@ bool fused_launch(const Plan& p, int logn, int64_t batch, int src, int dst, size
 // 384 tiles 52.1 / 47.8; FP32 2^15 640 tiles 66.7 / 67.2; FP64 2^16 640 tiles
 // 63.7 / 68.3; FP64 2^18 768 tiles 74.9 / 75.9, 640 tiles 67.2 / 64.1.  Real, both
 // directions: FP32 2^19 640 tiles 167 / 170 us; 2^20 640 tiles 201 / 196, 1184 317 /
-// 392; 2^21 640 tiles 227 / 204, 1184 361 / 392.
+// 392; 2^21 640 tiles 227 / 204, 1024 297 / 290, 1152 320 / 378; FP64 2^20 1024 262 / 259,
+// 1152 280 / 346.
 inline int64_t fused_min_tiles(bool f32, int logn, int form) {
+    if (form == FUSED_REAL && logn == (f32 ? 21 : 20)) return 1152;
     return (f32 ? form != FUSED_C2C && logn >= 20 : logn >= 18) ? 1024 : 640;
 }
 constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;

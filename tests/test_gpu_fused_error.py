@@ -58,7 +58,7 @@ def test_c2c_error(logn):
 def test_realft_error(logl):
     import torch
 
-    n, batch = 2 << logl, max(1, (1030 << 14) >> logl)
+    n, batch = 2 << logl, max(1, (1160 << 14) >> logl)
     x0 = torch.empty(n * batch, dtype=torch.float32, device="cuda")
     numrs_amd.gen_uniform(x0, 950 + logl)
     plan, one = numrs_amd.RealFTPlan("float32", n, batch), numrs_amd.RealFTPlan("float32", n, 1)

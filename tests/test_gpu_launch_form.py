@@ -34,7 +34,8 @@ def test_c2c(dtype):
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
 def test_realft(dtype):
     for logl in range(*RANGE[dtype]):
-        b = _batch(dtype, logl, 1024 if logl >= (20 if dtype == "float32" else 18) else 640)
+        late, last = (20, 21) if dtype == "float32" else (18, 20)
+        b = _batch(dtype, logl, 1152 if logl == last else 1024 if logl >= late else 640)
         at, below = (numrs_amd.RealFTPlan(dtype, 2 << logl, k) for k in (b, b - 1))
         for isign in (1, -1):
             info = at.launch_info(isign)
