@@ -103,6 +103,7 @@ int get_ctx(DeviceCtx** out) {
     hipLaunchKernelGGL(k_stage_twiddles, dim3(TW_STAGE_ELEMS / 256), dim3(256), 0, 0, c->c64s, c->c32s);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMalloc(&c->fs_pool, FS_POOL * sizeof(FsState)));
+    HIPCHK(hipMemset(c->fs_pool, 0, FS_POOL * sizeof(FsState)));
     HIPCHK(hipStreamCreateWithFlags(&c->fs_stream, hipStreamNonBlocking));
     c->fs_free.reserve(FS_POOL);
     for (int i = FS_POOL; i-- > 0;) c->fs_free.push_back(c->fs_pool + i);
@@ -118,20 +119,25 @@ static __global__ void k_state_zero(FsState* st) {
 }
 FsState* fs_state_take(DeviceCtx* ctx) {
     std::lock_guard<std::mutex> lk(g_ctx_mu);
-    if (ctx->fs_free.empty()) return nullptr;
-    FsState* st = ctx->fs_free.back();
-    hipLaunchKernelGGL(k_state_zero, dim3(1), dim3(256), 0, ctx->fs_stream, st);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->fs_stream) != hipSuccess) {
+    // (The clearing of those that were given back; done long ago as a rule.)
+    if (ctx->fs_free.empty() || hipStreamSynchronize(ctx->fs_stream) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
+    FsState* st = ctx->fs_free.back();
     ctx->fs_free.pop_back();
     return st;
 }
 void fs_state_give(int device, FsState* st) {
     std::lock_guard<std::mutex> lk(g_ctx_mu);
     auto it = g_ctx.find(device);
-    if (st && it != g_ctx.end()) it->second->fs_free.push_back(st);  // capacity reserved: does not throw
+    if (!st || it == g_ctx.end()) return;
+    int dev = device;
+    const bool other = hipGetDevice(&dev) == hipSuccess && dev != device;
+    if (other) (void)hipSetDevice(device);
+    hipLaunchKernelGGL(k_state_zero, dim3(1), dim3(256), 0, it->second->fs_stream, st);
+    if (hipGetLastError() == hipSuccess) it->second->fs_free.push_back(st);  // capacity reserved: does not throw
+    if (other) (void)hipSetDevice(dev);
 }
 
 int expired_check(uint32_t* d_word, hipStream_t s) {

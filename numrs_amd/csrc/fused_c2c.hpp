@@ -42,7 +42,7 @@
 // as it found it and needs no reset launch or memset before it.  (Launches of one
 // plan have equal grids.  If some overlapped against the rules, the very last group
 // still brings the count of those that have left to a multiple of the grid, finds
-// it unchanged and clears everything; a plan takes a state that is cleared first.)
+// it unchanged and clears everything; a state that a plan gives back is cleared.)
 #pragma once
 #include "pass_c2c.hpp"
 #include "real_fft.hpp"

@@ -239,9 +239,9 @@ inline int64_t fused_min_tiles(bool f32, int logn, int form) {
 constexpr size_t FUSED_RING_BYTES = size_t(192) << 20;
 bool plan_is_fused(const Plan& p);
 // A FsState of the current device's pool for a plan with fused launches (nullptr:
-// none left), cleared whatever its last plan left in it, and its return (when that
-// plan's launches are done: destroying a plan frees its workspace, which waits for
-// them).
+// none left), all zero, and its return, which clears it whatever the plan left in it
+// (when the plan's launches are done: destroying a plan frees its workspace, which
+// waits for them).
 FsState* fs_state_take(DeviceCtx* ctx);
 // Waits for the stream; NRFFT_E_HIP if the word is set, and clears it.
 int expired_check(uint32_t* d_word, hipStream_t s);

@@ -1,7 +1,7 @@
-"""GPU: a plan takes its counters cleared, whatever the plan that had them before
+"""GPU: a plan gets its counters cleared, whatever the plan that had them before
 left there (a caller that ran one plan on two streams at once must not spoil the
-plans of others).  The counters are overwritten by the host while no plan holds
-them."""
+plans of others).  The counters are overwritten by the host before their plan, which
+runs no more, is destroyed."""
 import ctypes
 
 import pytest
@@ -22,10 +22,10 @@ def test_counters_are_cleared_for_the_next_plan():
     word = plan.launch_info()["expired"]
     plan.execute(x, ref, 1)
     torch.cuda.synchronize()
-    plan.destroy()
     hip = ctypes.CDLL("libamdhip64.so.7")
     junk = (ctypes.c_uint32 * 96)(*([7] * 96))  # the flag, the tickets, the groups that have left: a line each
     assert hip.hipMemcpy(ctypes.c_void_p(word), junk, ctypes.c_size_t(ctypes.sizeof(junk)), 1) == 0
+    plan.destroy()
     plan = numrs_amd.C2CPlan("float32", [n], b)
     assert plan.launch_info()["expired"] == word  # the same counters
     plan.check()
