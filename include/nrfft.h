@@ -148,8 +148,8 @@ int nrfft_execute_correl(nrfft_plan plan, const void* d_data1, const void* d_dat
 /* Allocation-free batched four1 on device pointers.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Same transform, kernels and default tunings as nrfft_plan_c2c(dtype, {nn},
- * 1, batch) + nrfft_execute_c2c, but no plan: the four-step intermediate of
+ * Same transform and default tunings as nrfft_plan_c2c(dtype, {nn}, 1,
+ * batch) + nrfft_execute_c2c (same result up to rounding), but no plan: the four-step intermediate of
  * nn > 8192 lives in a 64 MiB device array built into the library (one per
  * GPU, held until the process ends), so nn * sizeof(complex) must not exceed
  * 64 MiB (FP32 nn <= 2^23, FP64 nn <= 2^22; larger -> NRFFT_E_UNSUPPORTED).

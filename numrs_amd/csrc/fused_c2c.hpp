@@ -341,7 +341,8 @@ struct FsEng {
 // away from them.
 // The table values are loaded before the last exchange and joined behind its
 // first barrier: loaded with the tile they took 32 registers through the first
-// stages (64 x 2^20 FP32 337 us against 324, FP64 2^19 and 2^20 spilled).
+// stages (64 x 2^20 FP32 337 us against 324; FP64 C2C 2^19 and 2^20 spilled).  All
+// a[h] from the tables: 2% less error in FP32, 2 to 4% more time.
 template <typename T, int S, int R, int BPT, int NB>
 struct FsTw {
     static_assert(R >= 8 && R % 8 == 0, "last radix 8, 16 or 32");
@@ -533,14 +534,18 @@ struct FsShape {
 // where they lie; the rows 0 and LA / 2 share a pair's place and are untangled
 // through the LDS.  RE = -1 takes column tiles likewise (columns n2 and LB - n2),
 // untangles before pass A, and pass B picks the columns up in their order.  So the
-// untangle costs no pass over memory.  64 x 2^19 reals FP32 (the data of 32 x 2^19
-// complex) forward 160 us, inverse 163, in passes 313 and 255; 37 x 2^20 134 and
-// 117 against 195 and 134.  What it pays instead: half as long runs in memory, one
-// of two at an odd element.
+// untangle costs no pass over memory.  64 x 2^19 reals FP32 forward 99 us, inverse
+// 98, in passes 158 and 129; 36 x 2^20 130 and 101 against 198 and 131.  What it pays
+// instead: half as long runs in memory, one of two at an odd element (11% of the
+// forward's write requests are below 64 bytes).
 //
 // RE = -2: the inverse of the correlation of the spectra `in` and `in2`: as RE = -1
 // on a conj(b) / N, taken where a tile is loaded (b in pieces of 8 values a thread;
 // more would not fit beside a).
+//
+// 128 registers a thread (two groups a CU).  The C2C forms keep to them; of the others
+// the FP32 inverses of 2^20 and 2^21 points spill 112 and 116 bytes a lane, the FP32
+// forwards from 2^18 and most FP64 ones 8 to 40.
 template <typename T, int S, int LA, int LB, int RE = 0>
 __global__ __attribute__((amdgpu_flat_work_group_size(FS_NT, FS_NT), amdgpu_waves_per_eu(4, 4))) void
 k_fused4(const cpx<T>* in, cpx<T>* out, cpx<T>* ring, FsState* st, FsDesc d, Twiddles<T> tw, const cpx<T>* in2,

@@ -173,7 +173,7 @@ void par_copy2d(char* dst, size_t dpitch, const char* src, size_t spitch, size_t
 //
 // What bounds them: the calls to the runtime.  Four hipMallocAsync and
 // hipFreeAsync take 65 us (2 KiB to 512 KiB), each transfer of pageable memory
-// about 12; so a lane's memory stays allocated, and small buffers move through
+// about 12; so a lane's memory stays allocated until lanes_trim, and small buffers move through
 // pinned memory by a copy kernel on the call's own stream (128 KiB in and out
 // around a kernel: 54 us against 64 by hipMemcpyAsync; 2 MiB: 227 and 225).  convlv
 // of 2^14 FP64 with 257 taps 122 -> 63 us (31 of them the kernel).

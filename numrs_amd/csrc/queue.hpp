@@ -20,9 +20,10 @@
 // Coherence across XCDs as in fused_c2c.hpp: SC1 stores and loads.
 //
 // What bounds it: as the fused four-step, the fabric between the XCDs and the
-// memory side.  500 items of mixed shapes, FP32 (914 MB): 583 us; as two launches,
+// memory side (2.1 times the algorithmic bytes pass it).  500 items of mixed shapes,
+// FP32 (914 MB): 583 us; as two launches,
 // one a pass with the whole intermediate in memory, 840 (HBM traffic twice).
-// 16 of 2048 x 2048 390 us against 575 (second-pass tiles of eight columns write
+// 16 of 2048 x 2048 382 us against 575 (second-pass tiles of eight columns write
 // 64-byte runs), 64 of 1024 x 1024 335 against 525.  Batches that are faster as two
 // launches (few tiles of long passes): queue_passes.hpp.
 //

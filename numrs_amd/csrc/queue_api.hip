@@ -299,6 +299,8 @@ static int build_uneven(UnevenState& u, const std::vector<int>* force_split = nu
         u.init[loaded] = (uint32_t)s.b.size();
         u.n1 += (int)s.a.size();
         u.n2 += (int)s.b.size();
+        // (A slab holds at most 64 items, none larger than those before, or one: its place
+        // held two or three slabs.)
         if (s.w1 - s.w0 > 64) return fail(NRFFT_E_UNSUPPORTED, "uneven ring order");
     }
     // One launch a pass if that is faster for most of the work.

@@ -324,8 +324,8 @@ int build_plan_real(Plan& p) {
             // plan holds both sequences, tagged by args[3] (1 = fwd only, -1 = inv only).
             size_t tmp = 0;
             use_c2c_tune(p, logl);
-            // Both passes and the untangle, of either direction, in one launch (37 x
-            // 2^20 reals FP32, both directions: 270 us against 370 in passes).
+            // Both passes and the untangle, of either direction, in one launch (36 x
+            // 2^20 reals FP32, both directions: 231 us against 330 in passes).
             Launch one;
             if (p.fused_ok && fused_launch(p, logl, batch, B_IN, B_OUT, FUSED_RING_BYTES, &one, &tmp, FUSED_REAL)) {
                 p.launches.push_back(one);
